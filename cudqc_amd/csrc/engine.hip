@@ -198,6 +198,10 @@ struct KParams {
     unsigned long long slice_ticks;  // > 0: time slice per launch in realtime-counter ticks (100 MHz)
     unsigned long long maxtot;  // largest task of the batch (~0ull: q->maxtot, device-resident steps)
     const int32_t* gbase;       // batched graphs: first id of each graph (multiples of 32); null = one graph
+    // bit rows of the two-hop, out- and in-lists (see bit_rows_kernel), rw words each; null =
+    // none kept for this graph
+    const uint32_t *b2, *bo, *bi;
+    int32_t rw;
 };
 
 // Id bitmaps (parent-live, parent-member, child-member, child-candidate, in-L(v),
@@ -205,11 +209,35 @@ struct KParams {
 // workgroup's HBM area. Either way they are all-zero between tasks: each branch and
 // task clears the words of the vertices it set.
 constexpr int NBITMAPS = 6;
+// Arrays of one word per 32 ids behind the chunked steps of a task (run_chunks), in the
+// workgroup's HBM area: the candidates passing the diameter pruning's degree test (pok), four
+// bit planes each of the candidates' out- and in-degree to the members, and the indices of
+// the words that hold a live id. The bitmaps are, like the others, all-zero between tasks.
+constexpr int PLANES = 4;
+constexpr int QUICK_MEMBERS = 14;  // most members: a child's member degrees fit 16 histogram bins
+constexpr int CHUNK_WORDS = 2 + 2 * PLANES;
+constexpr int CHUNK = 32;          // loop steps planned together
+constexpr int CHUNK_EVENTS = 80;   // candidates dropping out of pok within a chunk that LDS lists (others: gat, crit)
+enum StepBits : int { STEP_STOP = 1, STEP_SKIP = 2, STEP_LOOK = 4, STEP_BRANCH = 8, STEP_MEMBER = 16 };
+// LDS of a chunk, in the sort buffer (idle while a chunk is planned); the histograms of its
+// steps take the place of the member-degree histograms (16 + 16 bins per step).
+struct ChunkLds {
+    int32_t v[CHUNK + 1];      // v[i + 1]: the branch vertex of step i; v[i]: the vertex it removes
+    int32_t head[CHUNK];       // events of a step (linked lists)
+    int32_t ev_id[CHUNK_EVENTS];
+    int32_t ev_next[CHUNK_EVENTS];
+    uint4 md[QUICK_MEMBERS];   // the members' degrees at the chunk's start
+    uint32_t mo[QUICK_MEMBERS], mi[QUICK_MEMBERS];  // bit i: arc to / from the vertex step i removes
+    uint32_t vo[CHUNK], vi[CHUNK];                  // candidate degrees of step i's branch vertex at step i
+    uint32_t vm[CHUNK];                             // and its degrees to the members: out | in << 16
+    int32_t cls[CHUNK];        // StepBits
+};
 // LDS words of the live-set summary of the HBM-bitmap variant (it takes the LDS the
 // other variant gives its bitmaps): one bit per id up to 98,304 ids, per 2^s ids above
 constexpr int SUMW = 3072;
+static_assert(sizeof(ChunkLds) <= SORT_N * 8 && CHUNK * 32 <= 4 * (HMAX + 2), "chunk plan fits the idle LDS");
 struct Shared {
-    unsigned long long sortk[SORT_N];
+    alignas(16) unsigned long long sortk[SORT_N];
     int32_t ho[HMAX + 2], hi[HMAX + 2], so[HMAX + 2], si[HMAX + 2];
     int32_t cnt[12];
     int32_t red[12];
@@ -280,11 +308,22 @@ typedef const __attribute__((address_space(4))) KParams* KPtr;
 // run one task: a 256-thread workgroup, or one wavefront (64) for small tasks.
 template <int NT>
 struct W {
+    // The wavefront kernel runs tasks of a few dozen steps on small graphs, where planning
+    // chunks and reading whole rows costs more than it saves (0.24 ms against 0.17 ms of
+    // kernels on a 1,000-vertex graph): it walks lists, one step at a time.
+    static constexpr bool ROWS = NT > WAVE_T;
     KPtr P;
+    __device__ __forceinline__ bool rows() const { return ROWS && P->b2; }
     Shared* S;
     int tid;
     int kw;  // bitmap words in use
     uint32_t *plive, *pmem, *cmem, *ccand, *cL, *ccrit;  // id bitmaps (LDS or HBM)
+    // chunked steps: CHUNK_WORDS arrays of kw words from pok on (pok, the planes of the
+    // out-degrees to the members, those of the in-degrees, the indices of the nact words with
+    // a live id). planned: they are kept for the current task
+    uint32_t* pok;
+    bool planned;
+    int nact;
     // Batched graphs share one id space; a task's ids all lie in its graph's range
     // [gb, gb + kloc), and the id-indexed arrays and bitmaps are addressed relative to gb.
     uint32_t* vbase;   // the workgroup's id-indexed value arrays (graph-relative)
@@ -346,12 +385,16 @@ struct W {
         cur_gid = gid;
         gb = P->gbase ? P->gbase[gid] : 0;
         const long long k = P->kloc;
-        uint32_t* pr = vbase - 4ll * gb;          // parent degree records
-        uint32_t* cr = vbase + 4 * k - 4ll * gb;  // child degree records
-        pom = Field{pr}; poc = Field{pr + 1}; pim = Field{pr + 2}; pic = Field{pr + 3};
-        com = Field{cr}; coc = Field{cr + 1}; cim = Field{cr + 2}; cic = Field{cr + 3};
+        prec = (uint4*)vbase;
+        crec = (uint4*)(vbase + 4 * k);
+        bind_records();
         pl2 = vbase + 8 * k - gb;
         adjc = vbase + 9 * k - gb;
+    }
+    __device__ __forceinline__ void bind_records() {
+        uint32_t *pr = (uint32_t*)(prec - gb), *cr = (uint32_t*)(crec - gb);
+        pom = Field{pr}; poc = Field{pr + 1}; pim = Field{pr + 2}; pic = Field{pr + 3};
+        com = Field{cr}; coc = Field{cr + 1}; cim = Field{cr + 2}; cic = Field{cr + 3};
     }
     int dirty_m, dirty_l;  // child bitmaps: members mem[0..dirty_m) and lst[0..dirty_l) are set
     bool crit_marks;       // critical() ran: members and ccrit bits among lst too
@@ -393,11 +436,13 @@ struct W {
     }
     uint32_t cur_uid, cur_depth;  // the task being expanded (parent of the children written)
     uint32_t nbranch;             // branches run for the current task / piece
+    bool credit;                  // chunked steps: a stack check passed and no child was written since
     uint32_t launch_steps;        // stack checks this workgroup passed in this launch
     unsigned long long t_start;   // thread 0: realtime counter at the launch's start (time slices)
     bool discard_child;           // the current level-0 branch lies before root_first: it only
                                   // tells whether it writes a child (no child, clique or count)
-    Field pom, poc, pim, pic, com, coc, cim, cic;  // parent and child degrees (4 per id)
+    uint4 *prec, *crec;  // parent and child degree records, by graph-relative id
+    Field pom, poc, pim, pic, com, coc, cim, cic;  // their fields (4 per id)
     uint32_t *pl2, *adjc;
     int32_t *pids, *mem, *la, *lb, *lc, *lst, *crit, *gat;
     unsigned long long* hsort;  // HBM sort keys for children above SORT_N (2k entries)
@@ -607,8 +652,11 @@ struct W {
     }
     // reference inc/device_kernels.hpp:141-178 (d_vert_isextendable)
     __device__ __forceinline__ bool vert_ext(int w, int cs, int ub, int lb, int meo, int mei) const {
+        return degrees_ext(make_uint4(com[w], coc[w], cim[w], cic[w]), cs, ub, lb, meo, mei);
+    }
+    __device__ __forceinline__ bool degrees_ext(uint4 d, int cs, int ub, int lb, int meo, int mei) const {
         const int32_t *mdo = P->mdo, *mdi = P->mdi;
-        uint32_t om = com[w], oc = coc[w], im = cim[w], ic = cic[w];
+        const uint32_t om = d.x, oc = d.y, im = d.z, ic = d.w;
         if (om + oc < (uint32_t)meo) return false;
         if (im + ic < (uint32_t)mei) return false;
         if (om + oc < (uint32_t)gmd((int)(cs + oc), mdo)) return false;
@@ -679,15 +727,17 @@ struct W {
     // reference src/device_kernels.cu:1307-1486 (d_calculate_LU_bounds), with the
     // member scan on thread 0 and the candidate-prefix loops as parallel searches over
     // the sorted candidate member degrees (held as histograms in S->ho / S->hi).
-    __device__ __forceinline__ bool lu_bounds(int cm, int rc, int& ub, int& lb, int& meo, int& mei) {
+    // degrees(a) gives the four degrees of the child's member a.
+    template <class F>
+    __device__ __forceinline__ bool lu_bounds(int cm, int rc, int& ub, int& lb, int& meo, int& mei, F&& degrees) {
         const int32_t *mdo = P->mdo, *mdi = P->mdi;
         if (tid == 0) {
-            int x = mem[0];
-            int mino = (int)com[x], mino_c = (int)coc[x], sumo = (int)com[x], mint_o = (int)(com[x] + coc[x]);
-            int mini = (int)cim[x], mini_c = (int)cic[x], sumi = (int)cim[x], mint_i = (int)(cim[x] + cic[x]);
+            const uint4 x = degrees(0);
+            int mino = (int)x.x, mino_c = (int)x.y, sumo = (int)x.x, mint_o = (int)(x.x + x.y);
+            int mini = (int)x.z, mini_c = (int)x.w, sumi = (int)x.z, mint_i = (int)(x.z + x.w);
             for (int a = 1; a < cm; ++a) {
-                int y = mem[a];
-                uint32_t om = com[y], oc = coc[y], im = cim[y], ic = cic[y];
+                const uint4 y = degrees(a);
+                const uint32_t om = y.x, oc = y.y, im = y.z, ic = y.w;
                 sumo += (int)om;
                 if ((uint32_t)mino > om) { mino = (int)om; mino_c = (int)oc; }
                 else if ((uint32_t)mino == om) { if ((uint32_t)mino_c > oc) mino_c = (int)oc; }
@@ -746,6 +796,13 @@ struct W {
         if (cm + ub < P->min_size) return false;
         if (ub < 0 || ub < lb) return false;
         return true;
+    }
+
+    __device__ __forceinline__ bool lu_bounds(int cm, int rc, int& ub, int& lb, int& meo, int& mei) {
+        return lu_bounds(cm, rc, ub, lb, meo, mei, [&](int a) {
+            const int x = mem[a];
+            return make_uint4(com[x], coc[x], cim[x], cic[x]);
+        });
     }
 
     __device__ __forceinline__ void clear_hist(int cm) {
@@ -829,22 +886,83 @@ struct W {
         return c;
     }
 
+    // Lists (in crit) the bitmap words with a set bit of bmA or bmB (null: none) inside the task's id range, so
+    // that row words elsewhere are not read; returns their number.
+    __device__ __forceinline__ int list_words(const uint32_t* bmA, const uint32_t* bmB) {
+        const bool ranged = !(id_lo == INT_MIN && id_hi == INT_MAX);
+        const int w0 = ranged ? (id_lo - gb) >> 5 : 0, w1 = ranged ? (id_hi - 1 - gb) >> 5 : kw - 1;
+        if (tid == 0) S->cnt[11] = 0;
+        __syncthreads();
+        for (int w = w0 + tid; w <= w1; w += NT)
+            if (bmA[w] | (bmB ? bmB[w] : 0u)) crit[atomicAdd(&S->cnt[11], 1)] = w;
+        return read_counter(11);
+    }
+    // can-degrees of the listed vertices x = gat[0..n), counted on their bit rows: a wavefront
+    // keeps ROW_WORDS words per lane of the candidate bitmap in registers and streams the
+    // vertices' row words past them (a population count each, no lookup per list entry).
+    static constexpr int ROW_WORDS = 8;
+    __device__ __forceinline__ void recount_rows(int n, int nw) {
+        const int wave = tid >> 6, lane = tid & 63;
+        for (int t0 = 0; t0 < nw; t0 += 64 * ROW_WORDS) {
+            int w[ROW_WORDS];
+            uint32_t c[ROW_WORDS];
+            const int used = (min(nw - t0, 64 * ROW_WORDS) + 63) >> 6;  // words per lane in this round
+#pragma unroll
+            for (int u = 0; u < ROW_WORDS; ++u) {
+                const int t = t0 + u * 64 + lane;
+                w[u] = crit[min(t, nw - 1)];
+                c[u] = t < nw ? ccand[w[u]] : 0u;
+            }
+            for (int j = wave; j < n; j += NT / 64) {
+                const int x = gat[j];
+                const unsigned long long row = (unsigned long long)x * (unsigned long long)P->rw;
+                uint32_t o[ROW_WORDS], i[ROW_WORDS];
+#pragma unroll
+                for (int u = 0; u < ROW_WORDS; ++u) {
+                    o[u] = i[u] = 0;
+                    if (u < used) {
+                        o[u] = P->bo[row + w[u]];
+                        i[u] = P->bi[row + w[u]];
+                    }
+                }
+                uint32_t s = 0;  // out-count | in-count << 16 (at most 16,384 each in a round)
+#pragma unroll
+                for (int u = 0; u < ROW_WORDS; ++u) s += __popc(o[u] & c[u]) + (__popc(i[u] & c[u]) << 16);
+                s = wave_sum(s);
+                if (lane == 0) {
+                    coc[x] = (t0 ? coc[x] : 0u) + (s & 0xFFFFu);
+                    cic[x] = (t0 ? cic[x] : 0u) + (s >> 16);
+                }
+            }
+        }
+    }
+
     // can-degrees of live vertices recounted as |out(x) n R|, |in(x) n R| (R = ccand).
     // Each vertex is counted by a group of RG lanes (coalesced list reads, many vertices
-    // in flight); vertices with long lists (hubs) are queued and counted one per wavefront.
+    // in flight); vertices with long lists (hubs) are queued and counted one per wavefront,
+    // on their bit rows where those have fewer words than the lists have entries.
     __device__ __forceinline__ void recount(int cm, const int32_t* R, int nr) {
         constexpr unsigned long long LONG_LIST = 512;
         constexpr int RG = 8;
         const unsigned long long *oo = P->oo, *io = P->io;
         const int N = cm + nr;
-        if (tid == 0) S->cnt[8] = 0;
+        const int nw = rows() ? list_words(ccand, nullptr) : 0;
+        // lists longer than this are counted on rows (the bitmap lookup of a list entry costs
+        // an LDS access, or an HBM access for large graphs)
+        const unsigned long long row_list = !rows() ? ~0ull : lsum ? (unsigned long long)nw : 2ull * (unsigned long long)nw;
+        if (tid == 0) { S->cnt[8] = 0; S->cnt[11] = 0; }
         __syncthreads();
         const int sub = tid & (RG - 1);
         for (int i = tid / RG; i < N; i += NT / RG) {
             const int x = i < cm ? mem[i] : R[i - cm];
             const unsigned long long ob = oo[x], oe = oo[x + 1], ib = io[x], ie = io[x + 1];
-            if ((oe - ob) + (ie - ib) > LONG_LIST) {
-                if (sub == 0) gat[atomicAdd(&S->cnt[8], 1)] = x;
+            if (sub == 0) bytes += 4ull * ((oe - ob) + (ie - ib)) + 32;
+            const unsigned long long len = (oe - ob) + (ie - ib);
+            if (len > row_list || len > LONG_LIST) {  // rows from the front of gat, lists from its end
+                if (sub == 0) {
+                    if (len > row_list) gat[atomicAdd(&S->cnt[8], 1)] = x;
+                    else gat[N - 1 - atomicAdd(&S->cnt[11], 1)] = x;
+                }
                 continue;
             }
             const uint32_t co = count_cand_group<RG>(P->on, ob, oe, sub);
@@ -852,20 +970,19 @@ struct W {
             if (sub == 0) {
                 coc[x] = co;
                 cic[x] = ci;
-                bytes += 4ull * ((oe - ob) + (ie - ib)) + 32;
             }
         }
         __syncthreads();
-        const int nlong = S->cnt[8];
+        const int nrows = S->cnt[8], nlong = S->cnt[11];
         const int wave = tid >> 6, lane = tid & 63;
+        if (rows()) recount_rows(nrows, nw);
         for (int j = wave; j < nlong; j += NT / 64) {
-            const int x = gat[j];
+            const int x = gat[N - 1 - j];
             const uint32_t co = count_cand_wave(P->on, oo[x], oo[x + 1], lane);
             const uint32_t ci = count_cand_wave(P->in, io[x], io[x + 1], lane);
             if (lane == 0) {
                 coc[x] = co;
                 cic[x] = ci;
-                bytes += 4ull * ((oo[x + 1] - oo[x]) + (io[x + 1] - io[x])) + 32;
             }
         }
         __syncthreads();
@@ -873,14 +990,39 @@ struct W {
     // can-degrees of live vertices decremented by the arcs of dropped candidates
     __device__ __forceinline__ void decrement(const int32_t* D, int nd) {
         const unsigned long long *oo = P->oo, *io = P->io;
+        const int nw = rows() ? list_words(ccand, cmem) : 0;
+        if (rows()) {  // on bit rows: a thread owns 32 ids and adds up the dropped rows' words
+            for (int t = tid; t < nw; t += NT) {
+                const int w = crit[t];
+                const uint32_t live = ccand[w] | cmem[w];
+                for (int j0 = 0; j0 < nd; j0 += 31) {
+                    const int jn = min(31, nd - j0);
+                    uint32_t co[5] = {0, 0, 0, 0, 0}, ci[5] = {0, 0, 0, 0, 0};
+#pragma unroll 4
+                    for (int j = 0; j < jn; ++j) {
+                        const unsigned long long at = (unsigned long long)D[j0 + j] * (unsigned long long)P->rw + w;
+                        count_bits<5>(ci, P->bo[at] & live);
+                        count_bits<5>(co, P->bi[at] & live);
+                    }
+                    for (uint32_t m = co[0] | co[1] | co[2] | co[3] | co[4] | ci[0] | ci[1] | ci[2] | ci[3] | ci[4]; m;
+                         m &= m - 1) {
+                        const int bit = __builtin_ctz(m), x = gb + 32 * w + bit;
+                        coc[x] -= plane_value<5>(co, bit);
+                        cic[x] -= plane_value<5>(ci, bit);
+                    }
+                }
+            }
+        }
         for (int i = tid; i < nd; i += NT) {
             int u = D[i];
-            thread_scan_bits(P->on, oo[u], oo[u + 1], cmem, ccand, [&](int w, uint32_t m, uint32_t c) {
-                if (m | c) atomicSub(&cic[w], 1u);
-            });
-            thread_scan_bits(P->in, io[u], io[u + 1], cmem, ccand, [&](int w, uint32_t m, uint32_t c) {
-                if (m | c) atomicSub(&coc[w], 1u);
-            });
+            if (!rows()) {
+                thread_scan_bits(P->on, oo[u], oo[u + 1], cmem, ccand, [&](int w, uint32_t m, uint32_t c) {
+                    if (m | c) atomicSub(&cic[w], 1u);
+                });
+                thread_scan_bits(P->in, io[u], io[u + 1], cmem, ccand, [&](int w, uint32_t m, uint32_t c) {
+                    if (m | c) atomicSub(&coc[w], 1u);
+                });
+            }
             bytes += 4ull * ((oo[u + 1] - oo[u]) + (io[u + 1] - io[u])) + 32;
         }
         __syncthreads();
@@ -1243,7 +1385,9 @@ struct W {
     // decrements.
     __device__ __forceinline__ void flush_l2(int tot) {
         const int np = l2_tot - tot;
-        if (np > 0) {
+        if (ROWS && np > 0 && nact > 0) {
+            flush_l2_rows(tot, np);
+        } else if (np > 0) {
             if (tid == 0) S->cnt[10] = 0;
             __syncthreads();
             const int lane = tid & 63;
@@ -1265,6 +1409,69 @@ struct W {
         }
         l2_tot = tot;
     }
+    // flush_l2 on bit rows: a thread owns 32 ids, adds up the pending rows' words in bit
+    // planes (31 rows a round) and applies each id's count with one plain update.
+    __device__ __forceinline__ void flush_l2_rows(int tot, int np) {
+        const uint32_t* aw = pok + (CHUNK_WORDS - 1) * kw;
+        for (int t = tid; t < nact; t += NT) {
+            const int w = (int)aw[t];
+            const uint32_t live = plive[w] & ~pmem[w];
+            if (!live) continue;
+            for (int j0 = 0; j0 < np; j0 += 31) {
+                const int jn = min(31, np - j0);
+                uint32_t c[5] = {0, 0, 0, 0, 0};
+#pragma unroll 8
+                for (int j = 0; j < jn; ++j) {
+                    const int p = pids[tot + j0 + j];
+                    count_bits<5>(c, P->b2[(unsigned long long)p * (unsigned long long)P->rw + w] & live);
+                }
+                for (uint32_t m = c[0] | c[1] | c[2] | c[3] | c[4]; m; m &= m - 1) {
+                    const int bit = __builtin_ctz(m);
+                    pl2[gb + 32 * w + bit] -= plane_value<5>(c, bit);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // c (bit planes of 32 counters) += the bits of x
+    template <int N>
+    __device__ __forceinline__ static void count_bits(uint32_t (&c)[N], uint32_t x) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const uint32_t carry = c[q] & x;
+            c[q] ^= x;
+            x = carry;
+        }
+    }
+    template <int N>
+    __device__ __forceinline__ static uint32_t plane_value(const uint32_t (&c)[N], int bit) {
+        uint32_t r = 0;
+#pragma unroll
+        for (int q = 0; q < N; ++q) r |= ((c[q] >> bit) & 1u) << q;
+        return r;
+    }
+    // Sum over the wavefront, in every lane's copy of lane 63 (DPP: no LDS traffic).
+    __device__ __forceinline__ static uint32_t wave_sum(uint32_t x) {
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+        x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+        return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    }
+
+    // Lists the bitmap words that hold a live id (all that a row word can meet); returns
+    // their number.
+    __device__ __forceinline__ int list_live_words() {
+        uint32_t* aw = pok + (CHUNK_WORDS - 1) * kw;
+        if (tid == 0) S->cnt[11] = 0;
+        __syncthreads();
+        for (int w = ((id_lo - gb) >> 5) + tid; w <= (id_hi - 1 - gb) >> 5; w += NT)
+            if (plive[w]) aw[atomicAdd(&S->cnt[11], 1)] = (uint32_t)w;
+        return read_counter(11);
+    }
+
     // One wavefront: lvl2adj -= 1 for every live non-member in the list a[0, n), with
     // SCAN_UNR entries per lane and their bitmap words in flight per round.
     __device__ __forceinline__ void wave_decrement_l2(const int32_t* __restrict__ a, int n, int lane) {
@@ -1310,6 +1517,509 @@ struct W {
         return true;
     }
 
+    // ------------------------------------------------------------- chunked steps
+    // Up to CHUNK consecutive loop steps of a task are planned together, before any of them
+    // changes the task's state. Almost every branch of a large task ends at its first bound
+    // test (98.6% on the R-MAT 2^20 unit), and that test needs only counts over the
+    // candidates: those in v's two-hop row that still pass the degree test, by degree to the
+    // members and by v's arcs. Done one step after another, each step paid some twenty
+    // dependent memory round trips and a dozen barriers (12 us on a task of 1,000 vertices,
+    // 600 us with eight workgroups a CU on one of 5,000); planned together, a step is a pass
+    // over the words of three bit rows, with the next rows' loads in flight, and the chunk
+    // shares its barriers. What a step does is a matter of the vertices removed up to it,
+    // which are known in advance (the positions from the end), so the plan is exact:
+    //   STEP_STOP    a member falls short, or too few vertices remain: the loop ends
+    //   STEP_SKIP    the removal makes the branch vertex fall short: no branch
+    //   STEP_LOOK    no member (nor the branch vertex) rules lookahead out: test it in full
+    //   STEP_BRANCH  the branch passes its first bound test: run it
+    // Only steps with one of the last two bits need the task's state at that step; with none
+    // in the chunk, the state moves to the chunk's end in one go.
+    // Reference loop: src/device_kernels.cu:25-173, src/host_functions.cu:987-1134.
+
+    // Rows of the removed vertices: adds up each live vertex's arcs from and to them, writes
+    // its degrees after the chunk to the child records (whole, so that they can become the
+    // task's) and, for a plan of branches, notes at which step a candidate drops out of pok.
+    __device__ __forceinline__ void plan_removals(int c, bool removes, bool branches, uint32_t mo2, uint32_t mi2) {
+        ChunkLds* L = (ChunkLds*)S->sortk;
+        const uint32_t* aw = pok + (CHUNK_WORDS - 1) * kw;
+        const uint4* pr = prec - gb;
+        uint4* cr = crec - gb;
+        const int i0 = removes ? 0 : 1;
+        for (int t = tid; t < nact; t += NT) {
+            const int w = (int)aw[t];
+            const uint32_t live = plive[w];
+            if (!live) continue;
+            uint32_t co[6] = {0, 0, 0, 0, 0, 0}, ci[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 8
+            for (int i = i0; i < c; ++i) {
+                const unsigned long long at = (unsigned long long)L->v[i] * (unsigned long long)P->rw + w;
+                count_bits<6>(ci, P->bo[at] & live);  // arcs p -> x: in-degrees
+                count_bits<6>(co, P->bi[at] & live);  // arcs x -> p: out-degrees
+            }
+            const uint32_t cand = branches ? pok[w] : 0u;
+            for (uint32_t m = live; m;) {
+                int bit[4];
+                uint4 d[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    bit[q] = m ? __builtin_ctz(m) : -1;
+                    m &= m - 1;
+                    d[q] = pr[gb + 32 * w + max(bit[q], 0)];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (bit[q] < 0) continue;
+                    const int x = gb + 32 * w + bit[q];
+                    const uint32_t no = plane_value<6>(co, bit[q]), ni = plane_value<6>(ci, bit[q]);
+                    const bool drops = ((cand >> bit[q]) & 1u) && (no | ni) &&
+                                       (d[q].x + d[q].y - no < mo2 || d[q].z + d[q].w - ni < mi2);
+                    if (drops) {  // the first step after which its out- or in-degree is too small
+                        uint32_t o = d[q].x + d[q].y, n = d[q].z + d[q].w;
+                        int step = c - 1;
+                        for (int i = i0; i < c; ++i) {
+                            const unsigned long long at = (unsigned long long)L->v[i] * (unsigned long long)P->rw + w;
+                            o -= (P->bi[at] >> bit[q]) & 1u;
+                            n -= (P->bo[at] >> bit[q]) & 1u;
+                            if (o < mo2 || n < mi2) { step = i; break; }
+                        }
+                        const int e = atomicAdd(&S->cnt[11], 1), next = atomicExch(&L->head[step], e);
+                        if (e < CHUNK_EVENTS) {
+                            L->ev_id[e] = x;
+                            L->ev_next[e] = next;
+                        } else {
+                            gat[e - CHUNK_EVENTS] = x;
+                            crit[e - CHUNK_EVENTS] = next;
+                        }
+                    }
+                    d[q].y -= no;
+                    d[q].w -= ni;
+                    cr[x] = d[q];
+                }
+            }
+        }
+    }
+
+    // Arcs between the chunk's vertices and the members: a wavefront takes one member or
+    // branch vertex at a time, its low half the arcs to the removed vertices, its high half the
+    // arcs from them (one load a lane).
+    __device__ __forceinline__ void plan_arcs(int c, bool removes, int nm, uint32_t mo, uint32_t mi) {
+        ChunkLds* L = (ChunkLds*)S->sortk;
+        const int wave = tid >> 6, lane = tid & 63, i = lane & 31;
+        const uint4* pr = prec - gb;
+        const bool used = i < c && (removes || i > 0);
+        const int p = used ? L->v[i] - gb : 0;
+#pragma unroll 4
+        for (int u = wave; u < nm + c; u += NT / 64) {
+            const int x = u < nm ? pids[u] : L->v[u - nm + 1];
+            const uint32_t* row = (lane < 32 ? P->bo : P->bi) + (unsigned long long)x * (unsigned long long)P->rw;
+            const uint4 d = pr[x];
+            const unsigned long long m = __ballot(used && ((row[p >> 5] >> (p & 31)) & 1u));
+            const uint32_t to_p = (uint32_t)m, from_p = (uint32_t)(m >> 32);
+            if (lane == 0) {
+                if (u < nm) {
+                    L->md[u] = d;
+                    L->mo[u] = to_p;
+                    L->mi[u] = from_p;
+                } else {
+                    const int s = u - nm;
+                    const uint32_t upto = 0xFFFFFFFFu >> (31 - s);
+                    const uint32_t oc = d.y - __popc(to_p & upto), ic = d.w - __popc(from_p & upto);
+                    L->vo[s] = oc;
+                    L->vi[s] = ic;
+                    L->vm[s] = d.x | (d.z << 16);
+                    const bool skip = (((to_p >> s) & 1u) && d.x + oc < mo) || (((from_p >> s) & 1u) && d.z + ic < mi);
+                    L->cls[s] = skip ? STEP_SKIP : 0;
+                }
+            }
+        }
+    }
+
+    // Histograms of the steps' candidates (those left after diameter pruning) by degree to the
+    // child's members: population counts of v's two-hop row AND pok AND the planes, split by
+    // v's own arcs. A thread keeps its words' pok and planes while it walks the steps.
+    __device__ __forceinline__ void plan_counts(int c, bool removes, int nm) {
+        ChunkLds* L = (ChunkLds*)S->sortk;
+        const uint32_t* aw = pok + (CHUNK_WORDS - 1) * kw;
+        uint32_t* hist = (uint32_t*)S->ho;
+        const int lane = tid & 63;
+        constexpr int U = 2;
+        const int np = nm == 0 ? 0 : 32 - __clz(nm);  // planes in use
+        for (int t0 = 0; t0 < nact; t0 += U * NT) {
+            int w[U];
+            uint32_t pk[U], po[U][PLANES], pi[U][PLANES];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = t0 + u * NT + tid;
+                w[u] = (int)aw[min(t, nact - 1)];
+                pk[u] = t < nact ? pok[w[u]] : 0u;
+#pragma unroll
+                for (int q = 0; q < PLANES; ++q) {
+                    po[u][q] = q < np ? pok[(1 + q) * kw + w[u]] : 0u;
+                    pi[u][q] = q < np ? pok[(1 + PLANES + q) * kw + w[u]] : 0u;
+                }
+            }
+#pragma unroll 2
+            for (int s = 0; s < c; ++s) {
+                const int v = L->v[s + 1];
+                const unsigned long long row = (unsigned long long)v * (unsigned long long)P->rw;
+                uint32_t y[U], to_v[U], from_v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    y[u] = P->b2[row + w[u]];
+                    to_v[u] = P->bi[row + w[u]];
+                    from_v[u] = P->bo[row + w[u]];
+                }
+                auto drop = [&](int x) {
+                    const int xw = (x - gb) >> 5;
+#pragma unroll
+                    for (int u = 0; u < U; ++u)
+                        if (w[u] == xw) pk[u] &= ~(1u << (x & 31));
+                };
+                if (s > 0 || removes) drop(L->v[s]);
+                for (int e = L->head[s]; e >= 0; e = e < CHUNK_EVENTS ? L->ev_next[e] : crit[e - CHUNK_EVENTS])
+                    drop(e < CHUNK_EVENTS ? L->ev_id[e] : gat[e - CHUNK_EVENTS]);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    y[u] &= pk[u];
+                    if (w[u] == ((v - gb) >> 5)) y[u] &= ~(1u << (v & 31));
+                }
+                uint32_t any = 0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) any |= y[u];
+                if (__ballot(any != 0) == 0) continue;
+                for (int q = 0; q <= nm; ++q) {
+                    uint32_t no = 0, ni = 0;  // low half: without v's arc, high half: with it
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        uint32_t yo = y[u], yi = y[u];
+#pragma unroll
+                        for (int k = 0; k < PLANES; ++k) {
+                            if (k >= np) break;
+                            yo &= (q >> k) & 1 ? po[u][k] : ~po[u][k];
+                            yi &= (q >> k) & 1 ? pi[u][k] : ~pi[u][k];
+                        }
+                        no += __popc(yo & ~to_v[u]) + (__popc(yo & to_v[u]) << 16);
+                        ni += __popc(yi & ~from_v[u]) + (__popc(yi & from_v[u]) << 16);
+                    }
+                    no = wave_sum(no);
+                    ni = wave_sum(ni);
+                    if (lane == 0) {
+                        atomicAdd(&hist[32 * s + q], no & 0xFFFFu);
+                        atomicAdd(&hist[32 * s + q + 1], no >> 16);
+                        atomicAdd(&hist[32 * s + 16 + q], ni & 0xFFFFu);
+                        atomicAdd(&hist[32 * s + 17 + q], ni >> 16);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (t0 + u * NT + tid < nact) pok[w[u]] = pk[u];
+        }
+    }
+
+    // smallest i in [a, b] with pred(i), else b + 1 (a > b gives a), found by one wavefront
+    template <class F>
+    __device__ __forceinline__ static int wave_first(int a, int b, int lane, F pred) {
+        for (int base = a; base <= b; base += 64) {
+            const unsigned long long m = __ballot(base + lane <= b && pred(base + lane));
+            if (m) return base + __builtin_ctzll(m);
+        }
+        return a > b ? a : b + 1;
+    }
+    // largest i in [a, b] with pred(i), else a - 1
+    template <class F>
+    __device__ __forceinline__ static int wave_last(int a, int b, int lane, F pred) {
+        for (int top = b; top >= a; top -= 64) {
+            const unsigned long long m = __ballot(top - lane >= a && pred(top - lane));
+            if (m) return top - __builtin_ctzll(m);
+        }
+        return a - 1;
+    }
+    // Sum of the i largest of the values whose numbers are h[0..cm] (h[x] = how many are x).
+    __device__ __forceinline__ static int hist_top(const uint32_t* h, int cm, int i) {
+        int s = 0;
+        for (int x = cm; x > 0; --x) {
+            const int t = min(i, (int)h[x]);
+            s += t * x;
+            i -= t;
+        }
+        return s;
+    }
+
+    // lu_bounds and members_ext of step s's branch, by one wavefront: whether the first bound
+    // test passes (reference src/device_kernels.cu:1307-1486).
+    __device__ __forceinline__ bool plan_bounds(int s, int nm, int lane) {
+        const ChunkLds* L = (const ChunkLds*)S->sortk;
+        const uint32_t *ho = (const uint32_t*)S->ho + 32 * s, *hi = ho + 16;
+        const int32_t *mdo = P->mdo, *mdi = P->mdi;
+        const int cm = nm + 1;
+        const uint32_t upto = 0xFFFFFFFFu >> (31 - s);
+        const int v = L->v[s + 1] - gb;
+        // lane a < nm: member a's degrees at this step, with v's arcs moved; lane nm: v's own
+        uint4 d = make_uint4(0, 0, 0, 0);
+        if (lane < nm) {
+            d = L->md[lane];
+            d.y -= __popc(L->mo[lane] & upto);
+            d.w -= __popc(L->mi[lane] & upto);
+            const unsigned long long row = (unsigned long long)pids[lane] * (unsigned long long)P->rw;
+            const uint32_t a = (P->bo[row + (v >> 5)] >> (v & 31)) & 1u;  // arc member -> v
+            const uint32_t b = (P->bi[row + (v >> 5)] >> (v & 31)) & 1u;  // arc v -> member
+            d.x += a; d.y -= a; d.z += b; d.w -= b;
+        } else if (lane == nm) {
+            d = make_uint4(L->vm[s] & 0xFFFFu, L->vo[s], L->vm[s] >> 16, L->vi[s]);
+        }
+        auto at = [&](uint32_t x, int a) { return (uint32_t)__builtin_amdgcn_readlane((int)x, a); };
+        int mino = (int)at(d.x, 0), mino_c = (int)at(d.y, 0), sumo = mino;
+        int mini = (int)at(d.z, 0), mini_c = (int)at(d.w, 0), sumi = mini;
+        uint32_t mint_o = (uint32_t)(mino + mino_c), mint_i = (uint32_t)(mini + mini_c);
+        for (int a = 1; a < cm; ++a) {
+            const uint32_t om = at(d.x, a), oc = at(d.y, a), im = at(d.z, a), ic = at(d.w, a);
+            sumo += (int)om;
+            if ((uint32_t)mino > om) { mino = (int)om; mino_c = (int)oc; }
+            else if ((uint32_t)mino == om && (uint32_t)mino_c > oc) mino_c = (int)oc;
+            mint_o = min(mint_o, om + oc);
+            sumi += (int)im;
+            if ((uint32_t)mini > im) { mini = (int)im; mini_c = (int)ic; }
+            else if ((uint32_t)mini == im && (uint32_t)mini_c > ic) mini_c = (int)ic;
+            mint_i = min(mint_i, im + ic);
+        }
+        int rc = 0;
+        for (int q = 0; q <= cm; ++q) rc += (int)ho[q];
+        int ub, lb, meo = gmd(cm + 1, mdo), mei = gmd(cm + 1, mdi);
+        if (mino < mdo[cm] || mini < mdi[cm]) {
+            const int nmin = max(gmd(cm, mdo) - mino, gmd(cm, mdi) - mini);
+            const int no = wave_first(nmin, mino_c, lane, [&](int i) { return !(mino + i < mdo[cm + i]); });
+            if (mino + no < mdo[cm + no]) return false;
+            const int ni = wave_first(nmin, mini_c, lane, [&](int i) { return !(mini + i < mdi[cm + i]); });
+            if (mini + ni < mdi[cm + ni]) return false;
+            lb = max(no, ni);
+            ub = min(P->ubo[mint_o], P->ubi[mint_i]) + 1 - cm;
+            if (ub > rc) ub = rc;
+            if (lb < ub) {
+                const int i1 = wave_first(lb, ub - 1, lane, [&](int i) {
+                    const int so = hist_top(ho, cm, i), si = hist_top(hi, cm, i);
+                    return !(sumo + si < cm * mdo[cm + i] && sumi + so < cm * mdi[cm + i]);
+                });
+                {
+                    const int so = hist_top(ho, cm, i1), si = hist_top(hi, cm, i1);
+                    if (sumo + so < cm * mdo[cm + i1] && sumi + si < cm * mdi[cm + i1]) return false;
+                }
+                lb = i1;
+                const int t = wave_last(i1 + 1, ub, lane, [&](int i) {
+                    const int so = hist_top(ho, cm, i), si = hist_top(hi, cm, i);
+                    return sumo + si >= cm * mdo[cm + i] && sumi + so >= cm * mdi[cm + i];
+                });
+                const int tight = t >= i1 + 1 ? t : i1;
+                if (ub > tight) ub = tight;
+                if (lb > 1) { meo = gmd(cm + lb, mdo); mei = gmd(cm + lb, mdi); }
+            }
+        } else {
+            ub = rc;
+            lb = cm < P->min_size ? P->min_size - cm : 0;
+        }
+        if (cm + ub < P->min_size) return false;
+        if (ub < 0 || ub < lb) return false;
+        return __ballot(lane < cm && !degrees_ext(d, cm, ub, lb, meo, mei)) == 0;
+    }
+
+    // Plans the next c steps (tot: live vertices before them; removes: the first starts with a
+    // removal; branches: false for a split pass, which runs none). Leaves each step's
+    // StepBits in L->cls and the degrees after the chunk in the child records.
+    __device__ __forceinline__ void plan_chunk(int tot, int nm, int c, bool removes, bool branches) {
+        ChunkLds* L = (ChunkLds*)S->sortk;
+        const uint32_t mo = (uint32_t)gmd(nm + 1, P->mdo), mi = (uint32_t)gmd(nm + 1, P->mdi);
+        const uint32_t mo2 = (uint32_t)gmd(nm + 2, P->mdo), mi2 = (uint32_t)gmd(nm + 2, P->mdi);
+        const int r = removes ? 1 : 0, wave = tid >> 6, lane = tid & 63;
+        if (tid <= c) {
+            const int pos = tot - r - tid;  // v[0]: the first step's removed vertex (none: any id, unused)
+            L->v[tid] = pids[max(0, min(pos, tot - 1))];  // (a step past the last vertex is a STEP_STOP)
+        }
+        if (tid < CHUNK) L->head[tid] = -1;
+        if (tid == 0) S->cnt[11] = 0;
+        if (branches)
+            for (int i = tid; i < 32 * c; i += NT) ((uint32_t*)S->ho)[i] = 0;
+        __syncthreads();
+        plan_arcs(c, removes, nm, mo, mi);
+        plan_removals(c, removes, branches, mo2, mi2);
+        __syncthreads();
+        if (branches) {
+            plan_counts(c, removes, nm);
+            __syncthreads();
+        }
+        for (int s = wave; s < c; s += NT / 64) {
+            const uint32_t upto = 0xFFFFFFFFu >> (31 - s);
+            const int tot_s = tot - r - s;
+            const bool removal = s > 0 || removes;
+            const uint32_t lo = (uint32_t)gmd(tot_s, P->mdo), li = (uint32_t)gmd(tot_s, P->mdi);
+            // member `lane` falls short at this step's removal; it rules lookahead out
+            bool falls = false, witness = false;
+            if (lane < nm) {
+                const uint4 d = L->md[lane];
+                const uint32_t a = L->mo[lane], b = L->mi[lane];
+                const uint32_t o = d.x + d.y - __popc(a & upto), i = d.z + d.w - __popc(b & upto);
+                falls = removal && ((((a >> s) & 1u) && o < mo) || (((b >> s) & 1u) && i < mi));
+                witness = o < lo || i < li;
+            } else if (lane == nm) {
+                witness = (L->vm[s] & 0xFFFFu) + L->vo[s] < lo || (L->vm[s] >> 16) + L->vi[s] < li;
+            }
+            int cls = L->cls[s];
+            if (removal && tot_s < P->min_size) cls = STEP_STOP;
+            else if (__ballot(falls)) cls = STEP_STOP | STEP_MEMBER;
+            else if (!removal) cls &= ~STEP_SKIP;
+            if (!(cls & (STEP_STOP | STEP_SKIP))) {
+                if (!__ballot(witness)) cls |= STEP_LOOK;
+                if (branches && plan_bounds(s, nm, lane)) cls |= STEP_BRANCH;
+            }
+            if (lane == 0) L->cls[s] = cls;
+        }
+        __syncthreads();
+    }
+
+    // Applies the removals of steps [a, b) of a chunk (position base - i for step i): each
+    // wavefront walks one removed vertex's out- and in-lists at a time.
+    __device__ __forceinline__ void apply_removals(int base, int a, int b) {
+        if (a >= b) return;
+        for (int i = a + tid; i < b; i += NT) bcl(plive, pids[base - i]);
+        __syncthreads();
+        const int wave = tid >> 6, lane = tid & 63;
+        for (int i = a + wave; i < b; i += NT / 64) {
+            const int p = pids[base - i];
+#pragma unroll
+            for (int dir = 0; dir < 2; ++dir) {
+                const int32_t* l = dir ? P->in : P->on;
+                const unsigned long long* off = dir ? P->io : P->oo;
+                unsigned long long lb = off[p], le = off[p + 1];
+                if (le - lb >= 512) {
+                    lb = wave_lower_bound(l, lb, le, id_lo, lane);
+                    le = wave_lower_bound(l, lb, le, id_hi, lane);
+                }
+                for (unsigned long long e = lb + lane; e < le; e += 64) {
+                    const int x = l[e];
+                    if (bt(plive, x)) atomicSub(dir ? &poc[x] : &pic[x], 1u);
+                }
+            }
+        }
+        __syncthreads();
+    }
+
+    // The branch loop of a task, in planned chunks (see run_task for the loop itself).
+    __device__ __forceinline__ void run_chunks(const TaskDesc& d, int tot, int ncov, int expansions, bool split,
+                                               int chunk, bool remove_first, bool first_host_child, int step0) {
+        const int nm = d.nm, mode = d.mode;
+        bool removes = remove_first;
+        for (int j = ncov; j < expansions;) {
+            const int in_chunk = (j - ncov) % chunk;
+            int c = min(CHUNK, expansions - j);
+            bool first_check = false;
+            if (split) c = min(c, chunk - in_chunk);
+            if (split ? in_chunk == 0 : P->slice_ticks != 0 || launch_steps == 0) {
+                // a workgroup's first check of a launch asks for no margin, so it counts for this
+                // chunk's first step alone (that the launch moves on), like the first step of an
+                // unplanned task
+                first_check = launch_steps == 0;
+                const int low = stack_low();
+                credit = !low;
+                if (low) {
+                    defer(d, tot, removes, expansions - j, low, step0 + (j - ncov), first_host_child);
+                    return;
+                }
+            }
+            if (split && in_chunk == 0)
+                write_piece(d, tot, nm, mode, removes, min(chunk, expansions - j), false, j - ncov, false);
+            tick(0);
+            plan_chunk(tot, nm, c, removes, !split);
+            tick(1);
+            const int r = removes ? 1 : 0, lane = tid & 63;
+            const int cls = lane < c ? ((const ChunkLds*)S->sortk)->cls[lane] : 0;
+            const uint32_t stop = (uint32_t)__ballot(cls & STEP_STOP), skip = (uint32_t)__ballot(cls & STEP_SKIP);
+            const uint32_t look = (uint32_t)__ballot(cls & STEP_LOOK), run = (uint32_t)__ballot(cls & STEP_BRANCH);
+            const bool member_stop = stop && (__ballot(cls & STEP_MEMBER) >> __builtin_ctz(stop)) & 1u;
+            int end = stop ? __builtin_ctz(stop) : c;      // steps run
+            int removed_end = end + (member_stop ? 1 : 0);  // steps whose removal ran (for the byte count)
+            int done = 0;                                   // steps whose removal is applied to the state
+            bool over = stop != 0;
+            __syncthreads();  // (the plan's LDS is free from here on)
+            for (uint32_t m = look | run; m; m &= m - 1) {
+                const int f = __builtin_ctz(m);
+                if (f >= end) break;
+                // the state before step f, then its removal
+                const int first = r ? 0 : 1;
+                apply_removals(tot - r, max(done, first), f);
+                done = max(done, f);
+                int tf = tot - max(0, f - first);  // live vertices before step f's removal
+                if (first_check && f > 0) credit = false;
+                if (!split && !credit) {  // (a passed check lets this workgroup write one child)
+                    const int low = stack_low();
+                    credit = !low;
+                    first_check = false;
+                    if (low) {
+                        ptot = tf;
+                        defer(d, tf, f > 0 || removes, expansions - (j + f), low, step0 + (j + f - ncov), first_host_child);
+                        end = removed_end = f;
+                        over = true;
+                        break;
+                    }
+                }
+                apply_removals(tot - r, max(done, first), f + 1);
+                done = f + 1;
+                tf = tot - r - f;
+                tick(0);
+                const bool la = lookahead(tf, nm, tf - nm, mode);
+                tick(2);
+                if (la) {
+                    if (!split) emit_clique(pids, tf);  // the piece holding this step emits it
+                    end = f;
+                    removed_end = f + 1;
+                    over = true;
+                    break;
+                }
+                if (!split && ((run >> f) & 1u)) {
+                    const bool wrote = branch(tf, nm, mode, first_host_child);
+                    ++nbranch;
+                    tick(0);
+                    if (wrote) { first_host_child = false; credit = false; }
+                }
+            }
+            if (first_check) credit = false;
+            // counters of the steps: the branches that ended at their first bound test
+            const uint32_t below = end > 0 ? 0xFFFFFFFFu >> (32 - end) : 0u;
+            const uint32_t quick = split ? 0u : below & ~skip & ~run;
+            nbranch += __popc(quick);
+            if (tid == 0 && quick) atomicAdd(&P->g->branches, (unsigned long long)__popc(quick));
+            if (tid < c) {
+                const int vpos = tot - r - tid - 1;
+                if (tid < removed_end && (tid > 0 || removes)) {
+                    const int p = pids[vpos + 1];
+                    bytes += 4ull * ((P->oo[p + 1] - P->oo[p]) + (P->io[p + 1] - P->io[p]) + (P->to[p + 1] - P->to[p])) + 48;
+                }
+                if ((quick >> tid) & 1u) {
+                    const int v = pids[vpos];
+                    bytes += 4ull * ((P->to[v + 1] - P->to[v]) + (P->oo[v + 1] - P->oo[v]) + (P->io[v + 1] - P->io[v])) + 48;
+                }
+            }
+            if (over) return;
+            const int first = r ? 0 : 1;
+            if (done == 0) {  // no step needed the state: the degrees after the chunk become the task's
+                for (int i = first + tid; i < c; i += NT) bcl(plive, pids[tot - r - i]);
+                uint4* x = prec; prec = crec; crec = x;
+                bind_records();
+                __syncthreads();
+            } else {
+                apply_removals(tot - r, max(done, first), c);
+            }
+            tot = tot - r - (c - 1);
+            ptot = tot;
+            removes = true;
+            j += c;
+        }
+    }
+    // Pushes the rest of a task for a full stack (low 1) or an ended time slice (low 2).
+    __device__ __forceinline__ void defer(const TaskDesc& d, int tot, bool removes, int iters, int low, int step0,
+                                          bool first_host_child) {
+        write_piece(d, tot, d.nm, d.mode, removes, iters, low == 1, step0, d.mode == MODE_HOST_L0 && !first_host_child);
+        if (tid == 0) atomicAdd(low == 1 ? &P->g->pushbacks : &P->g->slices, 1ull);
+    }
+
     // One branch (reference src/device_kernels.cu:92-165 / src/host_functions.cu:1046-1133):
     // add the last candidate v, diameter + degree pruning, critical-vertex pruning, clique
     // check, child write. Only members and the candidates in L(v) are materialised: all
@@ -1335,9 +2045,21 @@ struct W {
         // candidates within two hops of v (the others fail diameter pruning), collected into
         // lst; their child degrees stay implicit (lazy_v)
         {
-            unsigned long long b = P->to[v], e = P->to[v + 1];
-            clip_live(P->tn, b, e);
-            wg_collect(P->tn, b, e, plive, pmem, v, lst, 3);
+            if (ROWS && nact > 0) {
+                const uint32_t* aw = pok + (CHUNK_WORDS - 1) * kw;
+                const uint32_t* row = P->b2 + (unsigned long long)v * (unsigned long long)P->rw;
+                for (int t = tid; t < nact; t += NT) {
+                    const int w = (int)aw[t];
+                    uint32_t m = row[w] & plive[w] & ~pmem[w];
+                    if (w == ((v - gb) >> 5)) m &= ~(1u << (v & 31));
+                    if (!m) continue;
+                    for (int at = atomicAdd(&S->cnt[3], __popc(m)); m; m &= m - 1) lst[at++] = gb + 32 * w + __builtin_ctz(m);
+                }
+            } else {
+                unsigned long long b = P->to[v], e = P->to[v + 1];
+                clip_live(P->tn, b, e);
+                wg_collect(P->tn, b, e, plive, pmem, v, lst, 3);
+            }
         }
         if (tid == 0) bytes += 4ull * (P->to[v + 1] - P->to[v]) + 16;
         vob = P->oo[v]; voe = P->oo[v + 1]; vib = P->io[v]; vie = P->io[v + 1];
@@ -1624,7 +2346,13 @@ struct W {
         cur_uid = d.uid;
         cur_depth = d.depth;
         nbranch = 0;
-        if (tid == 0) { S->idr[0] = INT_MAX; S->idr[1] = INT_MIN; }
+        // Steps are planned in chunks for tasks whose branches emit no clique when their first
+        // bound test fails (fewer members than the least clique) and whose member degrees fit
+        // the bit planes.
+        const bool try_plan = rows() && nm <= QUICK_MEMBERS && nm + 1 < P->min_size &&
+                              !(mode == MODE_HOST_L0 && P->root_first > 0);
+        const uint32_t mo2 = (uint32_t)gmd(nm + 2, P->mdo), mi2 = (uint32_t)gmd(nm + 2, P->mdi);
+        if (tid == 0) { S->idr[0] = INT_MAX; S->idr[1] = INT_MIN; S->red[9] = 0; }
         __syncthreads();
         int lo = INT_MAX, hi = INT_MIN;
         for (int i = tid; i < T; i += NT) {
@@ -1635,7 +2363,17 @@ struct W {
             pom[x] = r.out_mem; poc[x] = r.out_can; pim[x] = r.in_mem; pic[x] = r.in_can; pl2[x] = r.lvl2adj;
             bs(plive, x);
             if (lsum) mark_live(x);
-            if (i < nm) bs(pmem, x);
+            if (i < nm) {
+                bs(pmem, x);
+            } else if (try_plan) {
+                if (r.out_mem > (uint32_t)nm || r.in_mem > (uint32_t)nm) S->red[9] = 1;
+                if (r.out_mem + r.out_can >= mo2 && r.in_mem + r.in_can >= mi2) bs(pok, x);
+#pragma unroll
+                for (int q = 0; q < PLANES; ++q) {
+                    if ((r.out_mem >> q) & 1u) bs(pok + (1 + q) * kw, x);
+                    if ((r.in_mem >> q) & 1u) bs(pok + (1 + PLANES + q) * kw, x);
+                }
+            }
         }
         bytes += 24ull * T / NT + 1;
         ptot = l2_tot = T;  // no lvl2adj decrement pending
@@ -1644,6 +2382,8 @@ struct W {
         __syncthreads();
         id_lo = S->idr[0];
         id_hi = S->idr[1] + 1;
+        planned = try_plan && !S->red[9];  // (set: a degree to the members above their number)
+        nact = rows() ? list_live_words() : 0;
         int tot = T, nc = T - nm;
         int expansions = piece ? min(d.iters, nc) : nc;
         // a level-0 piece resumes its task's loop at step step0 (window bounds count from there)
@@ -1656,7 +2396,11 @@ struct W {
         const int chunk = split ? max(1, d.iters) : 1;
         const bool remove_first = piece && (d.flags & TF_REMOVE_FIRST);
         bool first_host_child = (mode == MODE_HOST_L0) && !(d.flags & TF_L1_DONE);
+        if (ROWS && planned)
+            run_chunks(d, tot, ncov, expansions, split, chunk, remove_first, first_host_child, step0);
+        else
         for (int j = ncov; j < expansions; ++j) {
+            credit = false;
             // The split pass writes only at chunk starts, so it checks the stack only there:
             // a deferred piece then takes the place of that chunk's piece and no step is
             // covered twice (a check inside a chunk would defer steps its piece already holds).
@@ -1714,6 +2458,10 @@ struct W {
             plive[wd] = 0; pmem[wd] = 0;
             if (lsum) lsum[((pids[i] - gb) >> gsh) >> 5] = 0;  // every set bit came from a pid
         }
+        if (try_plan)
+            for (int w = ((id_lo - gb) >> 5) + tid; w <= (id_hi - 1 - gb) >> 5; w += NT)
+#pragma unroll
+                for (int q = 0; q <= 2 * PLANES; ++q) pok[q * kw + w] = 0;
         __syncthreads();
     }
     // sets every summary word (all ones: any id may be live; zero: the all-clear state)
@@ -1725,8 +2473,11 @@ struct W {
 };
 
 // Register budget: DQC_WAVES_PER_EU asks the compiler for that many waves per SIMD.
+// Workgroup kernel: 4 waves (128 VGPRs). The planned steps keep rows of words in registers;
+// with 8 waves (64 VGPRs) they spill, and the R-MAT 2^18 unit takes 55 ms of kernels instead of
+// 47 (6 waves: 49, 5 waves: 47), with twice the per-workgroup scratch memory.
 #ifndef DQC_WAVES_PER_EU
-#define DQC_WAVES_PER_EU 8
+#define DQC_WAVES_PER_EU 4
 #endif
 // TPB threads per task (a 256-thread workgroup, or one wavefront) and LKW words per LDS
 // id bitmap (the LDS-bitmap variant covers condensed ids below 32 * LKW).
@@ -1773,6 +2524,9 @@ void expand_kernel(KParams P) {
     }
     const int bw = BIG ? w.kw : LKW;
     w.plive = bm; w.pmem = bm + bw; w.cmem = bm + 2 * bw; w.ccand = bm + 3 * bw; w.cL = bm + 4 * bw; w.ccrit = bm + 5 * bw;
+    w.pok = base + 22 * k + (BIG ? (unsigned long long)NBITMAPS * w.kw : 0ull);
+    w.planned = false;
+    w.nact = 0;
     w.dirty_m = 0;
     w.dirty_l = 0;
     w.crit_marks = false;
@@ -1781,6 +2535,7 @@ void expand_kernel(KParams P) {
     w.id_lo = INT_MIN; w.id_hi = INT_MAX;
     w.clip_pair = 0;
     w.launch_steps = 0;
+    w.credit = false;
     w.t_start = __builtin_amdgcn_s_memrealtime();
     w.discard_child = false;
     if (threadIdx.x == 0) { S.acc_bytes = 0; S.cnt[9] = 0; }
@@ -2119,6 +2874,50 @@ __global__ void refill_kernel(const TaskDesc* sp_desc, const dqc::TaskVertex* sp
     for (unsigned long long i = gid; i < vend - v0; i += gsz) dst_vtx[dst_v0 + i] = sp_vtx[v0 + i];
 }
 
+// Bit rows of CSR lists: bit x of row v (rw words, graph-relative ids) is set when x is in
+// v's list. Bound by reading the lists once and writing the rows once: one workgroup per
+// row gathers it in LDS and writes it out whole. A list that is not strictly ascending,
+// leaves its graph's id range or (no_self) holds the vertex itself raises *bad: no bit row
+// then says the same as the list.
+constexpr int ROW_TILE = 8192;  // words of a row gathered at a time (262,144 ids)
+__global__ __launch_bounds__(256) void bit_rows_kernel(const unsigned long long* __restrict__ off,
+                                                       const int32_t* __restrict__ nbr, int n,
+                                                       const int32_t* __restrict__ gbase, int ngraphs, int rw,
+                                                       bool no_self, uint32_t* __restrict__ rows, uint32_t* bad) {
+    __shared__ uint32_t tile[ROW_TILE];
+    const int tid = threadIdx.x;
+    for (int v = blockIdx.x; v < n; v += gridDim.x) {
+        int gb = 0;
+        if (gbase) {  // the last graph that starts at or before v
+            int lo = 0, hi = ngraphs;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (gbase[mid] <= v) lo = mid; else hi = mid;
+            }
+            gb = gbase[lo];
+        }
+        const unsigned long long b = off[v], e = off[v + 1];
+        uint32_t* row = rows + (unsigned long long)v * (unsigned long long)rw;
+        for (int t0 = 0; t0 < rw; t0 += ROW_TILE) {
+            const int nw = min(ROW_TILE, rw - t0);
+            for (int i = tid; i < nw; i += 256) tile[i] = 0;
+            __syncthreads();
+            for (unsigned long long i = b + tid; i < e; i += 256) {
+                const int x = nbr[i] - gb;
+                if (x < 0 || x >= 32 * rw || (no_self && x == v - gb) || (i > b && nbr[i - 1] >= nbr[i])) {
+                    *bad = 1;
+                    continue;
+                }
+                const int w = (x >> 5) - t0;
+                if (w >= 0 && w < nw) atomicOr(&tile[w], 1u << (x & 31));
+            }
+            __syncthreads();
+            for (int i = tid; i < nw; i += 256) row[t0 + i] = tile[i];
+            __syncthreads();
+        }
+    }
+}
+
 // Per-step outcome of the level-0 branch loop (reference src/host_functions.cu:1014-1044):
 // bit0 = the removal at this step skips the branch (success 2), bit1 = lookahead holds,
 // bit2 = fewer than min_size vertices remain (the loop stops). Uses the same counts as
@@ -2196,9 +2995,16 @@ struct dqc_handle {
     int32_t* d_ltn = nullptr;
     uint8_t* d_flags = nullptr;
     int32_t* d_split = nullptr;
+    uint32_t* d_rows = nullptr;  // bit rows of the two-hop, out- and in-lists (null: none kept)
+    int32_t rw = 0;              // words per bit row
     std::vector<std::vector<int32_t>> host_cliques;  // level-0 lookahead clique, if any
     uint32_t* d_scratch = nullptr;
     unsigned long long stride = 0;
+    bool unclean = false;  // a run ended with an error since the scratch bitmaps were cleared
+    // words of the bitmaps in a workgroup's scratch area
+    long long bitmap_words() const {
+        return (long long)((big ? NBITMAPS : 0) + CHUNK_WORDS) * ((kloc + 31) / 32);
+    }
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     dqc_stats st{};
@@ -2258,7 +3064,7 @@ void drop_graphs(dqc_handle* h) {
 
 void free_graph(dqc_handle* h) {
     void* gp[] = {h->d_oo, h->d_io, h->d_to, h->d_on, h->d_in, h->d_tn, h->d_scratch,
-                  h->d_lto, h->d_ltn, h->d_flags, h->d_split, h->d_gbase};
+                  h->d_lto, h->d_ltn, h->d_flags, h->d_split, h->d_gbase, h->d_rows};
     for (void* p : gp)
         if (p) {
             hipFree(p);
@@ -2269,6 +3075,7 @@ void free_graph(dqc_handle* h) {
     h->d_scratch = nullptr;
     h->d_lto = nullptr; h->d_ltn = nullptr; h->d_flags = nullptr; h->d_split = nullptr;
     h->d_gbase = nullptr;
+    h->d_rows = nullptr;
 }
 
 // Descriptor of a task pushed from the host, with the degree features the kernels
@@ -2428,6 +3235,53 @@ static unsigned long long scratch_slots(const dqc_handle* h) {
     return (unsigned long long)std::max(h->launch_wg, wave_ok(h) ? h->wave_wg : 0);
 }
 
+// Zeroes the bitmaps of every workgroup's scratch area (the id-indexed values and lists
+// before them are written before they are read).
+static bool clear_bitmaps(dqc_handle* h, const char* what) {
+    const size_t pitch = sizeof(uint32_t) * h->stride, at = sizeof(uint32_t) * 22ull * (size_t)h->kloc;
+    return hip_ok(h, hipMemset2D((char*)h->d_scratch + at, pitch, 0, sizeof(uint32_t) * (size_t)h->bitmap_words(),
+                                 (size_t)scratch_slots(h) + 1), what);
+}
+
+// Most memory the three sets of bit rows may take: 16 GiB, graphs of up to 214,000
+// condensed vertices (2.2 GB per set at 132,279).
+constexpr unsigned long long MAX_ROW_BYTES = 16ull << 30;
+
+// Bit rows of the uploaded graph's lists. Graphs whose rows would exceed MAX_ROW_BYTES (or
+// the free memory), and lists that are not strictly ascending, keep none: the kernels then
+// walk the lists. Neither do graphs all of whose tasks the wavefront kernel runs, which
+// walks lists (building rows made opening a 1,000-vertex graph 1.6 ms longer).
+static dqc_status build_rows(dqc_handle* h) {
+    h->rw = ((h->kloc + 31) / 32 + 3) & ~3;
+    const unsigned long long words = (unsigned long long)h->n * (unsigned long long)h->rw;
+    if (h->n == 0 || wave_resident(h) || 3 * words * sizeof(uint32_t) > MAX_ROW_BYTES) return DQC_OK;
+    void* q = nullptr;
+    if (hipMalloc(&q, (3 * words + 1) * sizeof(uint32_t)) != hipSuccess) {
+        (void)hipGetLastError();
+        return DQC_OK;
+    }
+    h->allocs.push_back(q);
+    h->d_rows = (uint32_t*)q;
+    uint32_t bad = 0, *d_bad = h->d_rows + 3 * words;
+    if (!hip_ok(h, hipMemcpy(d_bad, &bad, sizeof bad, hipMemcpyHostToDevice), "bit rows")) return DQC_E_HIP;
+    const int32_t* gb = h->ngraphs > 1 ? h->d_gbase : nullptr;
+    const int grid = std::min(h->n, 8192);
+    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_to, h->d_tn, h->n, gb, h->ngraphs, h->rw, false, h->d_rows, d_bad);
+    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_oo, h->d_on, h->n, gb, h->ngraphs, h->rw, true, h->d_rows + words, d_bad);
+    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_io, h->d_in, h->n, gb, h->ngraphs, h->rw, true, h->d_rows + 2 * words,
+                                                 d_bad);
+    if (!hip_ok(h, hipGetLastError(), "bit rows launch") ||
+        !hip_ok(h, hipMemcpyAsync(&bad, d_bad, sizeof bad, hipMemcpyDeviceToHost, h->stream), "bit rows") ||
+        !hip_ok(h, hipStreamSynchronize(h->stream), "bit rows"))
+        return DQC_E_HIP;
+    if (bad) {
+        hipFree(q);
+        h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), q), h->allocs.end());
+        h->d_rows = nullptr;
+    }
+    return DQC_OK;
+}
+
 // Uploads n ids' CSR lists; kloc is the largest vertex count of one graph (n itself for
 // a single graph; batched graphs share the id space with 32-aligned bases).
 static dqc_status upload_impl(dqc_handle* h, int32_t n, int32_t kloc, const uint64_t* out_off, const int32_t* out_nbr,
@@ -2472,17 +3326,17 @@ static dqc_status upload_impl(dqc_handle* h, int32_t n, int32_t kloc, const uint
     // per-workgroup scratch: 10k words of id-indexed values (parent and child degree
     // records of 4 words per id, lvl2adj, critical counts) + 8 lists of k entries, the
     // HBM sort area (2k 64-bit keys: a child has at most k vertices, padded to a power of
-    // 2) and, for large graphs, the six id bitmaps (all words even, so 8-byte aligned)
-    const unsigned long long kk = (unsigned long long)h->kloc, kwords = (kk + 31) / 32;
-    h->stride = 22ull * kk + (h->big ? (unsigned long long)NBITMAPS * kwords : 0ull);
-    h->stride += h->stride & 1ull;
+    // 2), for large graphs the six id bitmaps, and the quick branch test's bitmaps
+    const unsigned long long kk = (unsigned long long)h->kloc;
+    h->stride = 22ull * kk + (unsigned long long)h->bitmap_words();
+    h->stride = (h->stride + 3ull) & ~3ull;  // 16-byte aligned degree records
     // keep the scratch within 96 GiB (fewer resident workgroups for very large graphs)
     const unsigned long long cap_wg = (96ull << 30) / (h->stride * sizeof(uint32_t));
     h->launch_wg = (int)std::max<unsigned long long>(1, std::min<unsigned long long>(h->workgroups, cap_wg > 1 ? cap_wg - 1 : 1));
     h->st.workgroups = h->launch_wg;
     if (!dev_alloc(h, &h->d_scratch, h->stride * (size_t)(scratch_slots(h) + 1), "scratch alloc")) return DQC_E_HIP;
-    if (h->big && !hip_ok(h, hipMemset(h->d_scratch, 0, sizeof(uint32_t) * h->stride * (size_t)(h->launch_wg + 1)), "scratch clear"))
-        return DQC_E_HIP;
+    if (!clear_bitmaps(h, "scratch clear")) return DQC_E_HIP;
+    h->unclean = false;
     h->st.n_condensed = n;
     return size_buffers(h);
 }
@@ -2495,7 +3349,8 @@ dqc_status dqc_upload_graph(dqc_handle* h, int32_t n, const uint64_t* out_off, c
     if (!h || n < 0 || !out_off || !in_off || !two_off) return DQC_E_ARG;
     h->ngraphs = 1;
     h->gbase.assign(1, 0);
-    return upload_impl(h, n, n, out_off, out_nbr, in_off, in_nbr, two_off, two_nbr);
+    const dqc_status rc = upload_impl(h, n, n, out_off, out_nbr, in_off, in_nbr, two_off, two_nbr);
+    return rc == DQC_OK ? build_rows(h) : rc;
 }
 
 dqc_status dqc_upload_graph_batch(dqc_handle* h, int32_t ngraphs, const int32_t* nverts,
@@ -2543,7 +3398,7 @@ dqc_status dqc_upload_graph_batch(dqc_handle* h, int32_t ngraphs, const int32_t*
     if (!dev_alloc(h, &h->d_gbase, (size_t)ngraphs, "graph alloc") ||
         !hip_ok(h, hipMemcpy(h->d_gbase, base.data(), sizeof(int32_t) * ngraphs, hipMemcpyHostToDevice), "upload"))
         return DQC_E_HIP;
-    return DQC_OK;
+    return build_rows(h);
 }
 
 dqc_status dqc_set_tables(dqc_handle* h, const int32_t* md_out, const int32_t* md_in, const int32_t* ub_out,
@@ -2677,10 +3532,9 @@ dqc_status dqc_reset(dqc_handle* h) {
         return DQC_E_HIP;
     h->extra_tasks = 0;
     h->st.tasks_expanded = h->st.branches = h->st.raw_cliques = 0;
-    // a failed launch can leave id-bitmap bits set in the HBM variant
-    if (h->big && h->d_scratch &&
-        !hip_ok(h, hipMemset(h->d_scratch, 0, sizeof(uint32_t) * h->stride * (size_t)(h->launch_wg + 1)), "reset"))
-        return DQC_E_HIP;
+    // a failed launch can leave bits set in the bitmaps held in HBM
+    if (h->unclean && h->d_scratch && !clear_bitmaps(h, "reset")) return DQC_E_HIP;
+    h->unclean = false;
     return DQC_OK;
 }
 
@@ -2897,6 +3751,11 @@ static KParams make_params(dqc_handle* h, unsigned long long ntask) {
     P.log_cap = h->log_cap;
     P.kloc = h->kloc;
     P.gbase = h->d_gbase;
+    const unsigned long long words = (unsigned long long)h->n * (unsigned long long)h->rw;
+    P.b2 = h->d_rows;
+    P.bo = h->d_rows ? h->d_rows + words : nullptr;
+    P.bi = h->d_rows ? h->d_rows + 2 * words : nullptr;
+    P.rw = h->rw;
     P.max_depth = (uint32_t)std::max(0, h->cfg.max_depth);
     P.root_steps = std::max(0, h->cfg.root_branches);
     P.root_first = std::max(0, h->cfg.root_first);
@@ -3148,7 +4007,15 @@ static dqc_status resident_run(dqc_handle* h, int32_t sched, int64_t max_steps, 
     return DQC_OK;
 }
 
+static dqc_status run_loop(dqc_handle* h, int32_t sched, int64_t max_launches, int32_t* finished);
+
 static dqc_status run_launches(dqc_handle* h, int32_t sched, int64_t max_launches, int32_t* finished) {
+    const dqc_status rc = run_loop(h, sched, max_launches, finished);
+    if (rc != DQC_OK && h) h->unclean = true;
+    return rc;
+}
+
+static dqc_status run_loop(dqc_handle* h, int32_t sched, int64_t max_launches, int32_t* finished) {
     if (!h || sched < DQC_SCHED_DEFAULT || sched > DQC_SCHED_LEARNED) return DQC_E_ARG;
     if (sched == DQC_SCHED_DEFAULT) sched = h->cfg.schedule;
     if (!h->d_mdo || !h->d_oo) { h->err = "graph and tables must be set first"; return DQC_E_ARG; }
