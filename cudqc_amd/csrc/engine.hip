@@ -56,6 +56,7 @@ constexpr int HMAX = 256;          // member-degree histogram bins (members < HM
 constexpr int WAVE_T = 64;
 constexpr int WAVE_KW = 64;
 constexpr int WAVE_KMAX = WAVE_KW * 32;
+constexpr int LANE_TASK = 64;  // largest task whose vertices fit a wavefront's lanes (lane_task)
 // Split passes (the removal and lookahead steps of a task cut into pieces, one step after
 // another) run on workgroups of SPLIT_T threads: each step scans the removed vertex's
 // lists, and four times the lanes cut the memory round trips of a long list fourfold.
@@ -130,33 +131,36 @@ struct TaskLog {
 };
 static_assert(sizeof(TaskLog) == 36, "task log layout");
 
+// Counters that every task or child updates stand on 256 bytes of their own: updates of one
+// line are carried out one after another, and with all of them on one or two lines they were
+// what bounded the 256-graph batch (some nine updates per task of a few dozen microseconds).
 // Per-queue counters (one per task stack / stream).
 struct QCtr {
-    unsigned long long next_task;  // next work item of the current launch
-    unsigned long long sp_alloc;   // task stack top: (tasks << 34) | records
-    unsigned long long root_first; // level-0 split: (branch << 32) | stack index of the first child
+    alignas(256) unsigned long long next_task;  // next work item of the current launch
+    alignas(256) unsigned long long sp_alloc;   // task stack top: (tasks << 34) | records
+    alignas(256) unsigned long long pend;       // batch tasks not yet finished: (tasks << 34) | records
+    alignas(256) unsigned long long used;       // main + deferred: (tasks << 34) | records. Every push
+                                   // adds to it first and tests the capacity on the value it returns,
+                                   // so two regions can never be filled past each other
+    alignas(256) unsigned long long root_first; // level-0 split: (branch << 32) | stack index of the first child
     unsigned long long ntask;      // device-resident steps: tasks in the current batch
     unsigned long long first;      //   its first stack index
     unsigned long long v0;         //   and its first record
     unsigned long long maxtot;     //   and its largest task (the stack reserve is sized by it)
-    unsigned long long pend;       // batch tasks not yet finished: (tasks << 34) | records
     unsigned long long wg_limit;   // workgroups the stack has room for (device-resident steps)
     unsigned long long def_alloc;  // deferred region, growing down from the top of the stack
                                    // arrays: (pieces << 34) | records
-    unsigned long long used;       // main + deferred: (tasks << 34) | records. Every push adds
-                                   // to it first and tests the capacity on the value it returns,
-                                   // so two regions can never be filled past each other
     unsigned long long split_budget;  // device-resident steps: piece records the order kernel
                                       // may mark for splitting in the current batch
 };
 // Counters shared by every launch of a handle.
 struct GCtr {
-    unsigned long long clq_alloc;  // clique store: (sets << 40) | ids
-    unsigned long long tasks, branches, cliques, bytes, slow_sorts;
+    alignas(256) unsigned long long clq_alloc;  // clique store: (sets << 40) | ids
+    alignas(256) unsigned long long next_uid;   // task ids handed out (the level-0 task is id 0)
+    alignas(256) unsigned int error;            // read before every push and clique
+    alignas(256) unsigned long long tasks;
+    unsigned long long branches, cliques, bytes, slow_sorts;
     unsigned long long phase[8];   // realtime ticks per phase (profiling runs)
-    unsigned int error;
-    unsigned int pad;
-    unsigned long long next_uid;   // task ids handed out (the level-0 task is id 0)
     unsigned long long log_n;      // task-log records requested
     unsigned long long steps;      // device-resident steps that expanded a batch
     unsigned long long truncated;  // children not pushed: deeper than max_depth
@@ -201,7 +205,9 @@ struct KParams {
     // bit rows of the two-hop, out- and in-lists (see bit_rows_kernel), rw words each; null =
     // none kept for this graph
     const uint32_t *b2, *bo, *bi;
+    const uint32_t* rows_bad;   // set while the rows are built if no row stands for some list; null = checked
     int32_t rw;
+    int32_t tlen;               // entries of the md and ub tables
 };
 
 // Id bitmaps (parent-live, parent-member, child-member, child-candidate, in-L(v),
@@ -308,12 +314,13 @@ typedef const __attribute__((address_space(4))) KParams* KPtr;
 // run one task: a 256-thread workgroup, or one wavefront (64) for small tasks.
 template <int NT>
 struct W {
-    // The wavefront kernel runs tasks of a few dozen steps on small graphs, where planning
-    // chunks and reading whole rows costs more than it saves (0.24 ms against 0.17 ms of
-    // kernels on a 1,000-vertex graph): it walks lists, one step at a time.
+    // Tasks above 64 vertices on the wavefront kernel have a few dozen steps on a small graph,
+    // where planning chunks costs more than it saves: it walks lists, one step at a time.
     static constexpr bool ROWS = NT > WAVE_T;
     KPtr P;
-    __device__ __forceinline__ bool rows() const { return ROWS && P->b2; }
+    bool has_rows;     // the graph's bit rows are kept
+    bool lane_tables;  // the minimum-degree tables are in LDS (lane_task)
+    __device__ __forceinline__ bool rows() const { return ROWS && has_rows; }
     Shared* S;
     int tid;
     int kw;  // bitmap words in use
@@ -436,6 +443,17 @@ struct W {
     }
     uint32_t cur_uid, cur_depth;  // the task being expanded (parent of the children written)
     uint32_t nbranch;             // branches run for the current task / piece
+    // thread 0: counts of this launch, added to GCtr when the workgroup ends, and finished
+    // tasks not yet taken off QCtr::pend
+    unsigned long long n_tasks, n_branches, n_cliques, done_pend;
+    __device__ __forceinline__ void finish_task(unsigned long long records, bool now) {
+        done_pend += (1ull << CNT_SHIFT) | records;
+        if (now || (done_pend >> CNT_SHIFT) >= 8 || (done_pend & SIZE_MASK) >= 4096) flush_pend();
+    }
+    __device__ __forceinline__ void flush_pend() {
+        if (done_pend) atomicSub(&P->q->pend, done_pend);
+        done_pend = 0;
+    }
     bool credit;                  // chunked steps: a stack check passed and no child was written since
     uint32_t launch_steps;        // stack checks this workgroup passed in this launch
     unsigned long long t_start;   // thread 0: realtime counter at the launch's start (time slices)
@@ -1108,7 +1126,7 @@ struct W {
         for (int i = tid; i < len; i += NT) P->clq_ids[off + i] = ids[i];
         if (tid == 0) {
             P->clq_meta[idx] = (off << 24) | (unsigned long long)len;
-            atomicAdd(&P->g->cliques, 1ull);
+            ++n_cliques;
         }
         bytes += 4ull * len / NT + 1;
     }
@@ -1241,17 +1259,17 @@ struct W {
         return (long long)t;
     }
 
-    // Thread 0: room for one push of `recs` records, onto the main stack or (deferred)
+    // Thread 0: room for a push of `tasks` tasks of `recs` records in all, onto the main stack or (deferred)
     // the deferred region. The capacity is tested on the combined main + deferred use
     // that the one atomic on q->used returns, so concurrent pushes to the two regions
     // cannot both pass on a stale view of the other; only then is the slot taken in its
     // region. Returns the region's previous (tasks << 34) | records, or ~0ull when full
     // or after an error.
-    __device__ __forceinline__ unsigned long long reserve(bool deferred, unsigned long long recs) {
+    __device__ __forceinline__ unsigned long long reserve(bool deferred, unsigned long long recs, unsigned long long tasks = 1) {
         if (__atomic_load_n(&P->g->error, __ATOMIC_RELAXED)) return ~0ull;
-        const unsigned long long inc = (1ull << CNT_SHIFT) | recs;
+        const unsigned long long inc = (tasks << CNT_SHIFT) | recs;
         const unsigned long long u = atomicAdd(&P->q->used, inc);
-        if ((u >> CNT_SHIFT) + 1 > P->sp_cap_t || (u & SIZE_MASK) + recs > P->sp_cap_v) {
+        if ((u >> CNT_SHIFT) + tasks > P->sp_cap_t || (u & SIZE_MASK) + recs > P->sp_cap_v) {
             note_spill(u, recs | (deferred ? (1ull << 63) : 0ull));
             return ~0ull;
         }
@@ -1281,7 +1299,22 @@ struct W {
     // over: push the rest back onto the stack; never at a workgroup's first check).
     __device__ __forceinline__ int stack_low() {
         unsigned long long low = 0;
-        if (tid == 0) {
+        if (tid == 0) low = (unsigned long long)check_stack();
+        const int r = (int)bcast0(low);
+        if (!r) ++launch_steps;
+        return r;
+    }
+    __device__ __forceinline__ int check_stack() {  // one thread
+        int low = stack_state();
+        if (low == 1 && done_pend) {  // its own finished tasks still count as pending
+            flush_pend();
+            low = stack_state();
+        }
+        return low;
+    }
+    __device__ __forceinline__ int stack_state() const {
+        int low;
+        {
             const unsigned long long a = __atomic_load_n(&P->q->used, __ATOMIC_RELAXED);
             const unsigned long long pend = __atomic_load_n(&P->q->pend, __ATOMIC_RELAXED);
             const unsigned long long mt = P->maxtot == ~0ull ? P->q->maxtot : P->maxtot;
@@ -1294,9 +1327,7 @@ struct W {
                 __builtin_amdgcn_s_memrealtime() - t_start > P->slice_ticks)
                 low = 2;
         }
-        const int r = (int)bcast0(low);
-        if (!r) ++launch_steps;
-        return r;
+        return low;
     }
 
     // Pushes the current state of the task (live vertices in position order with their
@@ -1985,7 +2016,7 @@ struct W {
             const uint32_t below = end > 0 ? 0xFFFFFFFFu >> (32 - end) : 0u;
             const uint32_t quick = split ? 0u : below & ~skip & ~run;
             nbranch += __popc(quick);
-            if (tid == 0 && quick) atomicAdd(&P->g->branches, (unsigned long long)__popc(quick));
+            if (tid == 0) n_branches += (unsigned long long)__popc(quick);
             if (tid < c) {
                 const int vpos = tot - r - tid - 1;
                 if (tid < removed_end && (tid > 0 || removes)) {
@@ -2126,6 +2157,7 @@ struct W {
     // vertex (reference src/host_functions.cu:1386-1500, 1503-1559).
     __device__ __forceinline__ long long branch_root(int s, int k, const dqc::TaskVertex* root) {
         const int v = k - s - 1, tot = k - s;
+        lane_tables = false;
         ptot = l2_tot = tot;  // the values below are computed as of step s
         id_lo = INT_MIN; id_hi = INT_MAX;  // (the live set is [0, tot): scans test ids themselves)
         begin_child(1);
@@ -2199,7 +2231,7 @@ struct W {
         int nr = read_counter(4);
         int ub = 0, lbd = 0, meo = 0, mei = 0;
         int32_t* R = la;
-        if (tid == 0 && !discard_child) atomicAdd(&P->g->branches, 1ull);  // window branches only
+        if (tid == 0 && !discard_child) ++n_branches;  // window branches only
         tick(3);
         bool ok = degree_prune(cm, &R, &nr, tot - 1 - nm, ub, lbd, meo, mei, lb, lc);
         if (lazy_v >= 0) {  // (degree_prune materialized the degrees if it got past its first test)
@@ -2328,6 +2360,548 @@ struct W {
         return ok ? 1 : 0;
     }
 
+    // ------------------------------------------------- small tasks: a vertex per lane
+    // A task of at most 64 vertices runs on one wavefront with its whole state in registers:
+    // lane i holds the vertex at position i (id, degrees, lvl2adj) and, as 64-bit masks over
+    // the positions, its arcs and two-hop neighbours inside the task. Vertex sets are masks too,
+    // so a removal, a diameter or degree test is a handful of instructions and a ballot, a
+    // degree recount one population count, with no memory access between a task's records and
+    // its children. On the list-walking path a step of such a task is bound by the latency of
+    // some hundred dependent accesses to the workgroup's HBM arrays. On the 256-graph
+    // batch (5.1 M tasks, 15 vertices on average) the enumeration takes 0.143 s instead of 1.29 s.
+    // Same steps and results as run_task / branch (which cite the reference lines).
+    static constexpr int LANE_MD = 160;  // entries of each minimum-degree table kept in LDS
+    // Children and cliques of the wavefront kernel's small tasks collect in LDS and are pushed
+    // together: the shared counters take about 16 M updates a second each, whatever the number
+    // of wavefronts, and with one push per child and clique those updates bounded the launch
+    // (4 ms per 65,536 tasks). The records lie in the idle member histograms, the
+    // descriptors behind the degree tables.
+    static constexpr bool BUFFERED = NT == WAVE_T;
+    static constexpr int BUF_RECORDS = 4 * (HMAX + 2) / 6, BUF_TASKS = 14, BUF_IDS = 240, BUF_SETS = 15;
+    struct BufTask { int32_t tot, nm, mode; uint32_t parent; uint16_t depth, gid, dmin_o, dmax_o, dmin_i, dmax_i; };
+    static_assert(2 * LANE_MD * 4 + BUF_TASKS * sizeof(BufTask) <= SORT_N * 8, "tables and descriptors fit the sort buffer");
+    int32_t* cbuf;  // BUF_IDS clique ids, then BUF_SETS lengths (wavefront kernel)
+    int buf_records, buf_tasks, buf_ids, buf_sets;
+    int grant;  // what the last stack check lets the wavefront write: 0 nothing, 1 a child, 2 a bufferful
+    // Pushes the collected children (consecutive descriptors and records).
+    __device__ __forceinline__ void flush_children(int lane) {
+        if (buf_tasks == 0) return;
+        __syncthreads();
+        unsigned long long a = 0;
+        uint32_t uid = 0;
+        if (lane == 0) {
+            a = reserve(false, (unsigned long long)buf_records, (unsigned long long)buf_tasks);
+            if (a != ~0ull) uid = (uint32_t)atomicAdd(&P->g->next_uid, (unsigned long long)buf_tasks) + 1u;
+        }
+        a = first_lane64(a);
+        uid = first_lane(uid);
+        if (a != ~0ull) {
+            const unsigned long long t = a >> CNT_SHIFT, o = a & SIZE_MASK;
+            uint32_t* dst = (uint32_t*)(P->sp_vtx + o);
+            const uint32_t* src = (const uint32_t*)S->ho;
+            for (int i = lane; i < 6 * buf_records; i += 64) dst[i] = src[i];
+            const BufTask* bt_ = (const BufTask*)((const int32_t*)S->sortk + 2 * LANE_MD);
+            unsigned long long at = o;
+            for (int i = 0; i < buf_tasks; ++i) {
+                if (i == lane) {
+                    const BufTask b = bt_[i];
+                    TaskDesc c;
+                    c.off = at; c.tot = b.tot; c.nm = b.nm; c.ncov = 0; c.mode = b.mode;
+                    c.iters = b.tot - b.nm; c.flags = 0; c.step0 = 0;
+                    c.uid = uid + (uint32_t)i;
+                    c.parent = b.parent; c.depth = b.depth; c.gid = b.gid;
+                    c.dmin_o = b.dmin_o; c.dmax_o = b.dmax_o; c.dmin_i = b.dmin_i; c.dmax_i = b.dmax_i;
+                    P->sp_desc[t + i] = c;
+                }
+                at += (unsigned long long)bt_[i].tot;
+            }
+        }
+        __syncthreads();
+        buf_records = buf_tasks = 0;
+        grant = 0;
+    }
+    // Stores the collected cliques.
+    __device__ __forceinline__ void flush_cliques(int lane) {
+        if (buf_sets == 0) return;
+        __syncthreads();
+        unsigned long long a = 0;
+        if (lane == 0)
+            a = __atomic_load_n(&P->g->error, __ATOMIC_RELAXED) ? ~0ull
+                : atomicAdd(&P->g->clq_alloc, ((unsigned long long)buf_sets << CNT_SHIFT) | (unsigned long long)buf_ids);
+        a = first_lane64(a);
+        if (a != ~0ull) {
+            const unsigned long long idx = a >> CNT_SHIFT, off = a & SIZE_MASK;
+            if (idx + buf_sets > P->clq_cap_s || off + buf_ids > P->clq_cap_i) {
+                if (lane == 0) atomicOr(&P->g->error, (unsigned)ERR_CLIQUES);
+            } else {
+                for (int i = lane; i < buf_ids; i += 64) P->clq_ids[off + i] = cbuf[i];
+                unsigned long long at = off;
+                for (int i = 0; i < buf_sets; ++i) {
+                    const int len = cbuf[BUF_IDS + i];
+                    if (i == lane) P->clq_meta[idx + i] = (at << 24) | (unsigned long long)len;
+                    at += (unsigned long long)len;
+                }
+                n_cliques += lane == 0 ? (unsigned long long)buf_sets : 0ull;
+            }
+        }
+        __syncthreads();
+        buf_ids = buf_sets = 0;
+    }
+    __device__ __forceinline__ static unsigned long long lane_mask(unsigned long long x, int i) {
+        return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, i) |
+               ((unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), i) << 32);
+    }
+    __device__ __forceinline__ static uint32_t first_lane(uint32_t x) {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+    }
+    __device__ __forceinline__ static unsigned long long first_lane64(unsigned long long x) {
+        return (unsigned long long)first_lane((uint32_t)x) | ((unsigned long long)first_lane((uint32_t)(x >> 32)) << 32);
+    }
+    __device__ __forceinline__ static uint32_t wave_min(uint32_t x) {
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x111, 0xf, 0xf, false));
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x112, 0xf, 0xf, false));
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x114, 0xf, 0xf, false));
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x118, 0xf, 0xf, false));
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x142, 0xa, 0xf, false));
+        x = min(x, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x143, 0xc, 0xf, false));
+        return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    }
+    __device__ __forceinline__ static uint32_t wave_max(uint32_t x) { return ~wave_min(~x); }
+
+    // Minimum-degree tables in the (idle) sort buffer; lmd is gmd on them.
+    __device__ __forceinline__ void load_lane_tables(int lane) {
+        int32_t* t = (int32_t*)S->sortk;
+        const int last = P->tlen - 1;
+        for (int x = lane; x < LANE_MD; x += 64) {
+            t[x] = P->mdo[min(x, last)];
+            t[LANE_MD + x] = P->mdi[min(x, last)];
+        }
+        lane_tables = true;
+    }
+    __device__ __forceinline__ int lmd(int k, const int32_t* t) const { return t[k < P->min_size ? P->min_size : k]; }
+
+    // Degrees of a lane's vertex inside the child.
+    struct LaneDeg { uint32_t om, oc, im, ic; };
+    struct LaneBounds { int ub, lb, meo, mei; };
+
+    // Sum of the i largest of the values whose numbers are h (lane x: how many are x).
+    __device__ __forceinline__ static int lane_top(uint32_t h, int cm, int i) {
+        int s = 0;
+        for (int x = cm; x > 0; --x) {
+            const int t = min(i, __builtin_amdgcn_readlane((int)h, x));
+            s += t * x;
+            i -= t;
+        }
+        return s;
+    }
+    // lu_bounds over the members mask cmm and the candidates R (their degrees to the members
+    // are counted here).
+    __device__ __forceinline__ bool lane_lu(unsigned long long cmm, int cm, unsigned long long R, const LaneDeg& d, int lane,
+                                            LaneBounds& b) const {
+        const int32_t *mdo = (const int32_t*)S->sortk, *mdi = mdo + LANE_MD;
+        const bool in = (cmm >> lane) & 1ull, cand = (R >> lane) & 1ull;
+        const int rc = __popcll(R);
+        const uint32_t mino = wave_min(in ? d.om : ~0u), mini = wave_min(in ? d.im : ~0u);
+        b.meo = lmd(cm + 1, mdo);
+        b.mei = lmd(cm + 1, mdi);
+        if ((int)mino < mdo[cm] || (int)mini < mdi[cm]) {
+            const int mino_c = (int)wave_min(in && d.om == mino ? d.oc : ~0u);
+            const int mini_c = (int)wave_min(in && d.im == mini ? d.ic : ~0u);
+            const int no_ = (int)mino, ni_ = (int)mini;
+            const int nmin = max(lmd(cm, mdo) - no_, lmd(cm, mdi) - ni_);
+            const int no = wave_first(nmin, mino_c, lane, [&](int i) { return !(no_ + i < mdo[cm + i]); });
+            if (no_ + no < mdo[cm + no]) return false;
+            const int ni = wave_first(nmin, mini_c, lane, [&](int i) { return !(ni_ + i < mdi[cm + i]); });
+            if (ni_ + ni < mdi[cm + ni]) return false;
+            b.lb = max(no, ni);
+            const uint32_t mint_o = wave_min(in ? d.om + d.oc : ~0u), mint_i = wave_min(in ? d.im + d.ic : ~0u);
+            b.ub = min(P->ubo[mint_o], P->ubi[mint_i]) + 1 - cm;
+            if (b.ub > rc) b.ub = rc;
+            if (b.lb < b.ub) {
+                uint32_t ho = 0, hi = 0;
+                for (int x = 0; x <= cm; ++x) {
+                    const uint32_t co = (uint32_t)__popcll(__ballot(cand && d.om == (uint32_t)x));
+                    const uint32_t ci = (uint32_t)__popcll(__ballot(cand && d.im == (uint32_t)x));
+                    if (lane == x) { ho = co; hi = ci; }
+                }
+                const int sumo = (int)wave_sum(in ? d.om : 0u), sumi = (int)wave_sum(in ? d.im : 0u);
+                const int i1 = wave_first(b.lb, b.ub - 1, lane, [&](int i) {
+                    const int so = lane_top(ho, cm, i), si = lane_top(hi, cm, i);
+                    return !(sumo + si < cm * mdo[cm + i] && sumi + so < cm * mdi[cm + i]);
+                });
+                {
+                    const int so = lane_top(ho, cm, i1), si = lane_top(hi, cm, i1);
+                    if (sumo + so < cm * mdo[cm + i1] && sumi + si < cm * mdi[cm + i1]) return false;
+                }
+                b.lb = i1;
+                const int t = wave_last(i1 + 1, b.ub, lane, [&](int i) {
+                    const int so = lane_top(ho, cm, i), si = lane_top(hi, cm, i);
+                    return sumo + si >= cm * mdo[cm + i] && sumi + so >= cm * mdi[cm + i];
+                });
+                const int tight = t >= i1 + 1 ? t : i1;
+                if (b.ub > tight) b.ub = tight;
+                if (b.lb > 1) { b.meo = lmd(cm + b.lb, mdo); b.mei = lmd(cm + b.lb, mdi); }
+            }
+        } else {
+            b.ub = rc;
+            b.lb = cm < P->min_size ? P->min_size - cm : 0;
+        }
+        if (cm + b.ub < P->min_size) return false;
+        return !(b.ub < 0 || b.ub < b.lb);
+    }
+    // cand_valid / vert_ext on a lane's degrees
+    __device__ __forceinline__ bool lane_valid(const LaneDeg& d, int cs, const LaneBounds& b) const {
+        const int32_t *mdo = (const int32_t*)S->sortk, *mdi = mdo + LANE_MD;
+        const uint32_t o = d.om + d.oc, i = d.im + d.ic;
+        return o >= (uint32_t)b.meo && i >= (uint32_t)b.mei && o >= (uint32_t)lmd(cs + (int)d.oc + 1, mdo) &&
+               i >= (uint32_t)lmd(cs + (int)d.ic + 1, mdi) && d.om + (uint32_t)b.ub - 1u >= (uint32_t)mdo[cs + b.ub] &&
+               d.im + (uint32_t)b.ub - 1u >= (uint32_t)mdi[cs + b.ub] && o >= (uint32_t)lmd(cs + b.lb, mdo) &&
+               i >= (uint32_t)lmd(cs + b.lb, mdi);
+    }
+    __device__ __forceinline__ bool lane_ext(const LaneDeg& d, int cs, const LaneBounds& b) const {
+        const int32_t *mdo = (const int32_t*)S->sortk, *mdi = mdo + LANE_MD;
+        const uint32_t o = d.om + d.oc, i = d.im + d.ic;
+        return o >= (uint32_t)b.meo && i >= (uint32_t)b.mei && o >= (uint32_t)lmd(cs + (int)d.oc, mdo) &&
+               i >= (uint32_t)lmd(cs + (int)d.ic, mdi) && !(d.oc == 0 && d.om < (uint32_t)lmd(cs + 1, mdo)) &&
+               !(d.ic == 0 && d.im < (uint32_t)lmd(cs + 1, mdi)) && d.om + (uint32_t)b.ub >= (uint32_t)mdo[cs + b.ub] &&
+               d.im + (uint32_t)b.ub >= (uint32_t)mdi[cs + b.ub] && o >= (uint32_t)lmd(cs + b.lb, mdo) &&
+               i >= (uint32_t)lmd(cs + b.lb, mdi);
+    }
+    // degree_prune: R in, the candidates left out; out / in: the lane's arc masks.
+    __device__ __forceinline__ bool lane_prune(unsigned long long cmm, int cm, unsigned long long& R, int ccount, LaneDeg& d,
+                                               unsigned long long out, unsigned long long in, uint32_t lists, int lane,
+                                               LaneBounds& b) {
+        if (!lane_lu(cmm, cm, R, d, lane, b)) return false;
+        const bool member = (cmm >> lane) & 1ull;
+        if (__ballot(member && !lane_ext(d, cm, b))) return false;
+        unsigned long long kept = __ballot(((R >> lane) & 1ull) && lane_valid(d, cm, b));
+        unsigned long long dropped = R & ~kept;
+        R = kept;
+        int k = __popcll(R), nd = __popcll(dropped), removed = ccount - k;
+        bool all_mat = removed == nd;
+        while (k > 0 && removed > 0) {
+            // (recounting and decrementing give the same counts; the bytes are those of the
+            // lists the reference's choice scans)
+            const unsigned long long seen = cmm | R;
+            const unsigned long long scanned = all_mat && nd < k + cm ? dropped : seen;
+            if ((scanned >> lane) & 1ull) bytes += 4ull * lists + 32;
+            if ((seen >> lane) & 1ull) {
+                d.oc = (uint32_t)__popcll(out & R);
+                d.ic = (uint32_t)__popcll(in & R);
+            }
+            const bool cand = (R >> lane) & 1ull;
+            const unsigned long long valid = __ballot(cand && lane_valid(d, cm, b));
+            if (!lane_lu(cmm, cm, valid, d, lane, b)) return false;
+            if (__ballot(member && !lane_ext(d, cm, b))) return false;
+            kept = __ballot(cand && lane_valid(d, cm, b));
+            dropped = R & ~kept;
+            R = kept;
+            k = __popcll(R);
+            nd = removed = __popcll(dropped);
+            all_mat = true;
+        }
+        return true;
+    }
+    // emit_clique of the vertices in `set`, each at its rank
+    __device__ __forceinline__ void lane_emit(unsigned long long set, int rank, int32_t id, int lane) {
+        const int len = __popcll(set);
+        if constexpr (BUFFERED) {
+            if (buf_ids + len > BUF_IDS || buf_sets == BUF_SETS) flush_cliques(lane);
+            if ((set >> lane) & 1ull) {
+                cbuf[buf_ids + rank] = id;
+                bytes += 4;
+            }
+            if (lane == 0) cbuf[BUF_IDS + buf_sets] = len;
+            buf_ids += len;
+            ++buf_sets;
+            return;
+        }
+        unsigned long long a = 0;
+        if (lane == 0)
+            a = __atomic_load_n(&P->g->error, __ATOMIC_RELAXED) ? ~0ull
+                : atomicAdd(&P->g->clq_alloc, (1ull << CNT_SHIFT) | (unsigned long long)len);
+        a = first_lane64(a);
+        if (a == ~0ull) return;
+        const unsigned long long idx = a >> CNT_SHIFT, off = a & SIZE_MASK;
+        if (idx >= P->clq_cap_s || off + len > P->clq_cap_i) {
+            if (lane == 0) atomicOr(&P->g->error, (unsigned)ERR_CLIQUES);
+            return;
+        }
+        if ((set >> lane) & 1ull) {
+            P->clq_ids[off + rank] = id;
+            bytes += 4;
+        }
+        if (lane == 0) {
+            P->clq_meta[idx] = (off << 24) | (unsigned long long)len;
+            ++n_cliques;
+        }
+    }
+    // stack_low for one wavefront; sets grant
+    __device__ __forceinline__ int lane_low(int lane) {
+        uint32_t low = 0;
+        if (lane == 0) {
+            low = (uint32_t)check_stack();
+            if (BUFFERED && !low && stack_far()) low = 4;
+        }
+        low = first_lane(low);
+        // (a launch's first check asks for no margin: it counts for one step, see run_chunks)
+        grant = low == 4 ? 2 : low ? 0 : launch_steps ? 1 : -1;
+        if (low == 0 || low == 4) ++launch_steps;
+        return (int)(low & 3u);
+    }
+    // Room for a full buffer of children from every workgroup, besides what stack_state asks for.
+    __device__ __forceinline__ bool stack_far() const {
+        const unsigned long long a = __atomic_load_n(&P->q->used, __ATOMIC_RELAXED);
+        const unsigned long long pend = __atomic_load_n(&P->q->pend, __ATOMIC_RELAXED);
+        const unsigned long long mt = P->maxtot == ~0ull ? P->q->maxtot : P->maxtot;
+        const unsigned long long wg = P->maxtot == ~0ull ? P->q->wg_limit : gridDim.x;
+        return (a >> CNT_SHIFT) + wg * BUF_TASKS + (pend >> CNT_SHIFT) + 1 <= P->sp_cap_t &&
+               (a & SIZE_MASK) + wg * (BUF_RECORDS + mt) + (pend & SIZE_MASK) + (unsigned long long)P->kloc <= P->sp_cap_v;
+    }
+
+    // Whether run_task's task may run on lanes (every lane of the wavefront calls it): time-
+    // sliced launches do not (a launch of such tasks ends within a millisecond, the shortest
+    // slice, so there is nothing to slice; they keep the path whose slices are pinned).
+    __device__ __forceinline__ bool lane_task_ok(const TaskDesc& d) const {
+        return has_rows && !P->slice_ticks && d.tot <= LANE_TASK && !(d.flags & TF_SPLIT) && P->min_size < LANE_MD &&
+               !(d.mode == MODE_HOST_L0 && (P->root_first > 0 || P->root_steps > 0));
+    }
+
+    // One task of at most 64 vertices on the calling wavefront. Returns false, with nothing
+    // done, when a record holds degrees outside what the masks imply (tasks pushed by hand).
+    __device__ __forceinline__ bool lane_task(const TaskDesc& task, const dqc::TaskVertex* rv, int lane) {
+        const int T = task.tot, nm = task.nm, mode = task.mode;
+        const int ncov = mode == MODE_DEVICE ? 0 : task.ncov;
+        const bool piece = (task.flags & TF_PIECE) != 0, remove_first = piece && (task.flags & TF_REMOVE_FIRST);
+        const int gbase = P->gbase ? P->gbase[task.gid] : 0;
+        dqc::TaskVertex r{};
+        if (lane < T) r = rv[lane];
+        if (__ballot(lane < T && (max(max(r.out_mem, r.out_can), max(r.in_mem, r.in_can)) > 64u ||
+                                  (lane >= nm && max(r.out_mem, r.in_mem) > (uint32_t)nm))))
+            return false;
+        if (!lane_tables) load_lane_tables(lane);
+        const int32_t *mdo = (const int32_t*)S->sortk, *mdi = mdo + LANE_MD;
+        const int id = (int)r.id, rel = lane < T ? id - gbase : 0;
+        uint32_t om = r.out_mem, oc = r.out_can, im = r.in_mem, ic = r.in_can, l2 = r.lvl2adj;
+        // arcs and two-hop neighbours among the task's vertices: position j's row words at
+        // every lane's id, one ballot each (the rows of small graphs are one or two cache lines)
+        unsigned long long out = 0, in = 0, two = 0;
+        int below = 0;  // ids smaller than the lane's
+#pragma unroll 8
+        for (int j = 0; j < T; ++j) {
+            const int x = __builtin_amdgcn_readlane(id, j);
+            const unsigned long long at = (unsigned long long)x * (unsigned long long)P->rw + (unsigned long long)(rel >> 5);
+            const uint32_t wo = P->bo[at], wi = P->bi[at], wt = P->b2[at];
+            const unsigned long long mo_ = __ballot(lane < T && ((wo >> (rel & 31)) & 1u));
+            const unsigned long long mi_ = __ballot(lane < T && ((wi >> (rel & 31)) & 1u));
+            const unsigned long long mt_ = __ballot(lane < T && ((wt >> (rel & 31)) & 1u));
+            if (lane == j) { out = mo_; in = mi_; two = mt_; }
+            below += x < id ? 1 : 0;
+        }
+        // list lengths, for the byte count
+        uint32_t olen = 0, ilen = 0, tlen = 0;
+        if (lane < T) {
+            olen = (uint32_t)(P->oo[id + 1] - P->oo[id]);
+            ilen = (uint32_t)(P->io[id + 1] - P->io[id]);
+            tlen = (uint32_t)(P->to[id + 1] - P->to[id]);
+            bytes += 24;
+        }
+        cur_uid = task.uid;
+        cur_depth = task.depth;
+        nbranch = 0;
+        n_tasks += piece ? 0 : 1;
+        const unsigned long long M = nm >= 64 ? ~0ull : (1ull << nm) - 1ull;
+        int tot = T, nc = T - nm;
+        const int expansions = piece ? min(task.iters, nc) : nc;
+        const int step0 = piece ? task.step0 : 0;
+        bool first_host_child = mode == MODE_HOST_L0 && !(task.flags & TF_L1_DONE);
+        if (!BUFFERED) grant = 0;
+        for (int j = ncov; j < expansions; ++j) {
+            unsigned long long live = tot >= 64 ? ~0ull : (1ull << tot) - 1ull;
+            if (grant <= 0) {
+                const int low = lane_low(lane);
+                if (low) {
+                    unsigned long long a = 0;
+                    if (lane == 0) a = reserve(low == 1, (unsigned long long)tot);
+                    a = first_lane64(a);
+                    if (a != ~0ull) {
+                        const bool deferred = low == 1;
+                        const unsigned long long t = deferred ? P->sp_cap_t - 1 - (a >> CNT_SHIFT) : a >> CNT_SHIFT;
+                        const unsigned long long o =
+                            deferred ? P->sp_cap_v - (a & SIZE_MASK) - (unsigned long long)tot : a & SIZE_MASK;
+                        if (lane < tot) {
+                            P->sp_vtx[o + lane] = dqc::TaskVertex{(uint32_t)id, om, oc, im, ic, l2};
+                            bytes += 24;
+                        }
+                        if (lane == 0) {
+                            TaskDesc p = task;
+                            p.off = o; p.tot = tot; p.nm = nm; p.ncov = 0; p.mode = mode;
+                            p.iters = expansions - j;
+                            p.flags = TF_PIECE | (j != ncov || remove_first ? TF_REMOVE_FIRST : 0) |
+                                      (mode == MODE_HOST_L0 && !first_host_child ? TF_L1_DONE : 0);
+                            p.step0 = step0 + (j - ncov);
+                            P->sp_desc[t] = p;
+                        }
+                    }
+                    if (lane == 0) atomicAdd(low == 1 ? &P->g->pushbacks : &P->g->slices, 1ull);
+                    break;
+                }
+            }
+            if (j != ncov || remove_first) {  // remove_one
+                --nc;
+                --tot;
+                if (tot < P->min_size) break;
+                const int p = tot;
+                live &= ~(1ull << p);
+                const uint32_t mo = (uint32_t)lmd(nm + 1, mdo), mi = (uint32_t)lmd(nm + 1, mdi);
+                const bool alive = (live >> lane) & 1ull;
+                const bool to = alive && ((lane_mask(out, p) >> lane) & 1ull), from = alive && ((lane_mask(in, p) >> lane) & 1ull);
+                ic -= to ? 1u : 0u;
+                oc -= from ? 1u : 0u;
+                if (alive && lane >= nm && ((lane_mask(two, p) >> lane) & 1ull)) --l2;
+                const unsigned long long bad = __ballot((to && im + ic < mi) || (from && om + oc < mo));
+                if (lane == p) bytes += 4ull * (olen + ilen + tlen) + 48;
+                if (bad & M) break;
+                if ((bad >> (tot - 1)) & 1ull) continue;
+            }
+            const bool alive = (live >> lane) & 1ull;
+            {  // lookahead
+                const uint32_t mo = (uint32_t)lmd(tot, mdo), mi = (uint32_t)lmd(tot, mdi);
+                const uint32_t l2min = mode == MODE_DEVICE ? (uint32_t)(nc - 1) : (uint32_t)(tot - 1);
+                if (!__ballot(alive && (om + oc < mo || im + ic < mi || (lane >= nm && l2 < l2min)))) {
+                    lane_emit(live, lane, id, lane);
+                    break;
+                }
+            }
+            // branch
+            const int v = tot - 1;
+            ++nbranch;
+            if (lane == v) bytes += 4ull * (olen + ilen + tlen) + 48;
+            int cm = nm + 1;
+            unsigned long long cmm = M | (1ull << v);
+            const unsigned long long out_v = lane_mask(out, v), in_v_ = lane_mask(in, v);
+            LaneDeg d{om, oc, im, ic};
+            if (alive) {
+                const uint32_t a = (uint32_t)((in_v_ >> lane) & 1ull), b = (uint32_t)((out_v >> lane) & 1ull);
+                d = LaneDeg{om + a, oc - a, im + b, ic - b};
+            }
+            const uint32_t mo2 = (uint32_t)lmd(nm + 2, mdo), mi2 = (uint32_t)lmd(nm + 2, mdi);
+            const unsigned long long hop = lane_mask(two, v) & live & ~cmm;
+            unsigned long long R = __ballot(((hop >> lane) & 1ull) && d.om + d.oc >= mo2 && d.im + d.ic >= mi2);
+            LaneBounds b{0, 0, 0, 0};
+            int state = lane_prune(cmm, cm, R, tot - 1 - nm, d, out, in, olen + ilen, lane, b) ? 1 : -1;
+            unsigned long long K = 0;
+            if (state == 1) {  // critical: 2 = failure, 0 = the second pruning failed
+                const bool member = (cmm >> lane) & 1ull;
+                const bool co = member && d.om + d.oc == (uint32_t)mdo[cm + b.lb] && d.oc > 0u;
+                const bool ci = member && d.im + d.ic == (uint32_t)mdi[cm + b.lb] && d.ic > 0u;
+                if (co) bytes += 4ull * olen + 16;
+                if (ci) bytes += 4ull * ilen + 16;
+                const unsigned long long mco = __ballot(co), mci = __ballot(ci);
+                K = __ballot(((R >> lane) & 1ull) && ((in & mco) | (out & mci)));
+                const int nk = __popcll(K);
+                if (nk > 0) {
+                    int adj = 0;
+                    for (unsigned long long m = K; m; m &= m - 1)
+                        adj += (int)((lane_mask(two, __builtin_ctzll(m)) >> lane) & 1ull);
+                    const bool crit = (K >> lane) & 1ull;
+                    if (crit) bytes += 4ull * (tlen + olen + ilen) + 48;
+                    if (__ballot((member && adj != nk) || (crit && adj < nk - 1))) {
+                        if (crit) bytes -= 4ull * (olen + ilen) + 32;  // (a failure ends the branch before these lists)
+                        state = 2;
+                    } else {
+                        if (((cmm | R) >> lane) & 1ull) {
+                            const uint32_t a = (uint32_t)__popcll(out & K), c = (uint32_t)__popcll(in & K);
+                            d.om += a; d.oc -= a; d.im += c; d.ic -= c;
+                        }
+                        const int nrest = __popcll(R & ~K);
+                        R = __ballot((((R & ~K) >> lane) & 1ull) && adj == nk);
+                        cmm |= K;
+                        cm += nk;
+                        state = lane_prune(cmm, cm, R, nrest, d, out, in, olen + ilen, lane, b) ? 1 : 0;
+                    }
+                }
+            }
+            // members in the order parent's, v, critical (of the child's records and a clique)
+            const int rank_m = lane < nm ? lane : lane == v ? nm : nm + 1 + __popcll(K & ((1ull << lane) - 1ull));
+            if (state >= 0 ? state != 2 : (mode == MODE_DEVICE || P->host_addfail)) {  // check_clique
+                const bool member = (cmm >> lane) & 1ull;
+                if (cm >= P->min_size && !__ballot(member && (d.om < (uint32_t)mdo[cm] || d.im < (uint32_t)mdi[cm])))
+                    lane_emit(cmm, rank_m, id, lane);
+            }
+            if (state != 1 || R == 0) continue;
+            // write_child
+            const unsigned long long set = cmm | R;
+            const int N = __popcll(set), child_mode = first_host_child ? MODE_HOST_L1 : MODE_DEVICE;
+            if (P->max_depth && cur_depth + 1u > P->max_depth) {
+                if (lane == 0) atomicAdd(&P->g->truncated, 1ull);
+                continue;
+            }
+            const bool mine = (set >> lane) & 1ull;
+            // enumeration order: members first, then min(mem), min(can), lvl2adj and id, all
+            // descending; the rank is the number of smaller keys
+            const unsigned long long key = ((unsigned long long)((R >> lane) & 1ull) << 56) |
+                                           ((unsigned long long)(127u - min(d.om, d.im)) << 48) |
+                                           ((unsigned long long)(127u - min(d.oc, d.ic)) << 40) |
+                                           ((unsigned long long)(uint32_t)~l2 << 8) | (unsigned long long)(63 - below);
+            int rank = 0;
+            for (unsigned long long m = set; m; m &= m - 1) rank += lane_mask(key, __builtin_ctzll(m)) < key ? 1 : 0;
+            const uint32_t od = d.om + d.oc, di = d.im + d.ic;
+            const uint32_t omin = wave_min(mine ? od : ~0u), omax = wave_max(mine ? od : 0u);
+            const uint32_t imin = wave_min(mine ? di : ~0u), imax = wave_max(mine ? di : 0u);
+            if (mine) bytes += 24;
+            if constexpr (BUFFERED) {
+                if (buf_records + N > BUF_RECORDS || buf_tasks == BUF_TASKS) {
+                    const int g = grant;  // (of this step's check, for the child at hand)
+                    flush_children(lane);
+                    grant = g == 2 ? 1 : g;
+                }
+                uint32_t* rec = (uint32_t*)S->ho + 6 * (buf_records + rank);
+                if (mine) { rec[0] = (uint32_t)id; rec[1] = d.om; rec[2] = d.oc; rec[3] = d.im; rec[4] = d.ic; rec[5] = l2; }
+                if (lane == 0)
+                    ((BufTask*)((int32_t*)S->sortk + 2 * LANE_MD))[buf_tasks] =
+                        BufTask{N, cm, child_mode, cur_uid, (uint16_t)min(cur_depth + 1u, 65535u), task.gid,
+                                (uint16_t)omin, (uint16_t)omax, (uint16_t)imin, (uint16_t)imax};
+                buf_records += N;
+                ++buf_tasks;
+                if (grant != 2) flush_children(lane);
+            } else {
+                unsigned long long a = 0;
+                if (lane == 0) a = reserve(false, (unsigned long long)N);
+                a = first_lane64(a);
+                if (a == ~0ull) continue;
+                const unsigned long long t = a >> CNT_SHIFT, o = a & SIZE_MASK;
+                if (mine) P->sp_vtx[o + rank] = dqc::TaskVertex{(uint32_t)id, d.om, d.oc, d.im, d.ic, l2};
+                if (lane == 0) {
+                    TaskDesc c;
+                    c.off = o; c.tot = N; c.nm = cm; c.ncov = 0; c.mode = child_mode;
+                    c.iters = N - cm; c.flags = 0; c.step0 = 0;
+                    c.uid = (uint32_t)(atomicAdd(&P->g->next_uid, 1ull) + 1);
+                    c.parent = cur_uid;
+                    c.depth = (uint16_t)min(cur_depth + 1u, 65535u); c.gid = task.gid;
+                    c.dmin_o = (uint16_t)omin; c.dmax_o = (uint16_t)omax;
+                    c.dmin_i = (uint16_t)imin; c.dmax_i = (uint16_t)imax;
+                    P->sp_desc[t] = c;
+                }
+                grant = 0;
+            }
+            first_host_child = false;
+        }
+        n_branches += (unsigned long long)nbranch;
+        if (P->log && lane == 0) {
+            const unsigned long long li = atomicAdd(&P->g->log_n, 1ull);
+            if (li < P->log_cap) {
+                TaskLog l;
+                l.uid = task.uid; l.parent = task.parent; l.depth = task.depth; l.nm = nm; l.tot = T;
+                l.dmin_o = task.dmin_o; l.dmax_o = task.dmax_o; l.dmin_i = task.dmin_i; l.dmax_i = task.dmax_i;
+                l.branches = nbranch; l.flags = (uint32_t)task.flags;
+                P->log[li] = l;
+            }
+        }
+        if (lane == 0) finish_task((unsigned long long)T, false);
+        return true;
+    }
+
     // ---------------------------------------------------------------- one task
     // reference src/device_kernels.cu:25-173 (device levels) and
     // src/host_functions.cu:987-1134 (host levels 0 and 1)
@@ -2342,6 +2916,7 @@ struct W {
         const int T = d.tot, nm = d.nm, mode = d.mode;
         const int ncov = mode == MODE_DEVICE ? 0 : d.ncov;
         const bool piece = (d.flags & TF_PIECE) != 0;
+        lane_tables = false;  // (the sort buffer is used)
         set_graph(d.gid);
         cur_uid = d.uid;
         cur_depth = d.depth;
@@ -2377,7 +2952,7 @@ struct W {
         }
         bytes += 24ull * T / NT + 1;
         ptot = l2_tot = T;  // no lvl2adj decrement pending
-        if (tid == 0 && !piece) atomicAdd(&P->g->tasks, 1ull);
+        if (tid == 0 && !piece) ++n_tasks;
         if (lo <= hi) { atomicMin(&S->idr[0], lo); atomicMax(&S->idr[1], hi); }
         __syncthreads();
         id_lo = S->idr[0];
@@ -2451,7 +3026,7 @@ struct W {
                 P->log[li] = r;
             }
         }
-        if (tid == 0) atomicSub(&P->q->pend, (1ull << CNT_SHIFT) | (unsigned long long)T);
+        if (tid == 0) finish_task((unsigned long long)T, true);
         if (lsum) __syncthreads();  // every test of the summary is done before it clears
         for (int i = tid; i < T; i += NT) {
             const int wd = (pids[i] - gb) >> 5;
@@ -2462,7 +3037,22 @@ struct W {
             for (int w = ((id_lo - gb) >> 5) + tid; w <= (id_hi - 1 - gb) >> 5; w += NT)
 #pragma unroll
                 for (int q = 0; q <= 2 * PLANES; ++q) pok[q * kw + w] = 0;
+        for (int t = tid; t < nact; t += NT) pok[(CHUNK_WORDS - 1) * kw + t] = 0;
         __syncthreads();
+    }
+    __device__ __forceinline__ void flush_buffers() {
+        if constexpr (BUFFERED) {
+            flush_children(tid);
+            flush_cliques(tid);
+            grant = 0;
+        }
+    }
+    // After lane_task on the first wavefront: what the other wavefronts have to know.
+    __device__ __forceinline__ bool leave_lanes(bool done) {
+        const unsigned long long x = bcast0(((unsigned long long)launch_steps << 1) | (done ? 1ull : 0ull));
+        launch_steps = (uint32_t)(x >> 1);
+        credit = false;
+        return x & 1ull;
     }
     // sets every summary word (all ones: any id may be live; zero: the all-clear state)
     __device__ __forceinline__ void fill_live_summary(uint32_t v) {
@@ -2524,7 +3114,15 @@ void expand_kernel(KParams P) {
     }
     const int bw = BIG ? w.kw : LKW;
     w.plive = bm; w.pmem = bm + bw; w.cmem = bm + 2 * bw; w.ccand = bm + 3 * bw; w.cL = bm + 4 * bw; w.ccrit = bm + 5 * bw;
-    w.pok = base + 22 * k + (BIG ? (unsigned long long)NBITMAPS * w.kw : 0ull);
+    w.pok = base + P.stride - (unsigned long long)CHUNK_WORDS * w.kw;  // (at the area's end)
+    w.has_rows = P.b2 && !(P.rows_bad && *P.rows_bad);
+    w.lane_tables = false;
+    w.grant = w.buf_records = w.buf_tasks = w.buf_ids = w.buf_sets = 0;
+    w.cbuf = nullptr;
+    if constexpr (W<TPB>::BUFFERED) {
+        __shared__ int32_t clique_buf[W<TPB>::BUF_IDS + W<TPB>::BUF_SETS];
+        w.cbuf = clique_buf;
+    }
     w.planned = false;
     w.nact = 0;
     w.dirty_m = 0;
@@ -2534,17 +3132,25 @@ void expand_kernel(KParams P) {
     w.lazy_v = -1;
     w.id_lo = INT_MIN; w.id_hi = INT_MAX;
     w.clip_pair = 0;
+    w.n_tasks = w.n_branches = w.n_cliques = w.done_pend = 0;
     w.launch_steps = 0;
     w.credit = false;
     w.t_start = __builtin_amdgcn_s_memrealtime();
     w.discard_child = false;
     if (threadIdx.x == 0) { S.acc_bytes = 0; S.cnt[9] = 0; }
     __syncthreads();
+    const unsigned long long ntask = P.in_ntask == ~0ull ? P.q->ntask : P.in_ntask;
+    // work items are taken 4 at a time while there are plenty of them for every wavefront
+    const unsigned long long take = TPB == WAVE_T && ntask >= 16ull * gridDim.x ? 4 : 1;
+    unsigned long long t = 0, t_end = 0;
     while (true) {
-        unsigned long long t = 0;
-        if (threadIdx.x == 0) t = atomicAdd(&P.q->next_task, 1ull);
-        t = w.bcast0(t);
-        if (t >= (P.in_ntask == ~0ull ? P.q->ntask : P.in_ntask)) break;
+        if (t == t_end) {
+            if (threadIdx.x == 0) t = atomicAdd(&P.q->next_task, take);
+            t = w.bcast0(t);
+            if (t >= ntask) break;
+            t_end = min(t + take, ntask);
+        }
+        const unsigned long long item = t++;
         if (P.split_s) {
             const TaskDesc d = P.in_desc[0];
             w.set_graph(d.gid);
@@ -2552,19 +3158,35 @@ void expand_kernel(KParams P) {
             w.cur_depth = d.depth;
             // level-0 branches keep no live bitmap (the live set is an id range)
             if constexpr (BIG) w.fill_live_summary(~0u);
-            w.discard_child = P.split_s[t] < P.root_first;
-            w.branch_root(P.split_s[t], d.tot, P.in_vtx + d.off);
+            w.discard_child = P.split_s[item] < P.root_first;
+            w.branch_root(P.split_s[item], d.tot, P.in_vtx + d.off);
             w.discard_child = false;
             if constexpr (BIG) w.fill_live_summary(0u);
         } else {
-            TaskDesc d = P.in_desc[t];
-            w.run_task(d, P.in_vtx + d.off);
+            const TaskDesc d = P.in_desc[item];
+            bool done = false;
+            if constexpr (TPB <= NT) {
+                if (w.lane_task_ok(d)) {
+                    if (threadIdx.x < 64) done = w.lane_task(d, P.in_vtx + d.off, threadIdx.x);
+                    if constexpr (TPB > 64) done = w.leave_lanes(done);
+                    w.tick(1);
+                }
+            }
+            if (!done) {
+                w.flush_buffers();  // (they lie in LDS that run_task uses)
+                w.run_task(d, P.in_vtx + d.off);
+            }
         }
     }
+    w.flush_buffers();
     atomicAdd(&S.acc_bytes, w.bytes);
     __syncthreads();
     if (threadIdx.x == 0) {
         atomicAdd(&P.g->bytes, S.acc_bytes);
+        if (w.n_tasks) atomicAdd(&P.g->tasks, w.n_tasks);
+        if (w.n_branches) atomicAdd(&P.g->branches, w.n_branches);
+        if (w.n_cliques) atomicAdd(&P.g->cliques, w.n_cliques);
+        w.flush_pend();
         if (P.profile) {
             w.tick(0);
             for (int i = 0; i < 8; ++i) atomicAdd(&P.g->phase[i], w.ph[i]);
@@ -2596,9 +3218,10 @@ constexpr int POP_T = 1024;
 __global__ __launch_bounds__(POP_T) void pop_kernel(PopParams pp) {
     __shared__ int first_bad;
     __shared__ unsigned maxtot;
-    const QCtr qv = *pp.q;
-    const unsigned long long st_t = qv.sp_alloc >> CNT_SHIFT, st_v = qv.sp_alloc & SIZE_MASK;
-    const unsigned long long df_t = qv.def_alloc >> CNT_SHIFT, df_v = qv.def_alloc & SIZE_MASK;
+    const unsigned long long sp = pp.q->sp_alloc, def = pp.q->def_alloc;
+    const unsigned long long st_t = sp >> CNT_SHIFT, st_v = sp & SIZE_MASK;
+    const unsigned long long df_t = def >> CNT_SHIFT, df_v = def & SIZE_MASK;
+    __syncthreads();  // (thread 0 writes both below)
     const bool from_main = st_t > 0;
     const unsigned long long avail = from_main ? st_t : df_t;
     const unsigned long long m = avail < pp.pool_tasks ? avail : pp.pool_tasks;
@@ -2874,18 +3497,30 @@ __global__ void refill_kernel(const TaskDesc* sp_desc, const dqc::TaskVertex* sp
     for (unsigned long long i = gid; i < vend - v0; i += gsz) dst_vtx[dst_v0 + i] = sp_vtx[v0 + i];
 }
 
+// Words [from, stride) of every workgroup's scratch area set to zero (one area a workgroup).
+__global__ __launch_bounds__(256) void clear_kernel(uint32_t* scratch, unsigned long long stride, unsigned long long from) {
+    uint32_t* area = scratch + (unsigned long long)blockIdx.x * stride;
+    for (unsigned long long i = from + threadIdx.x; i < stride; i += 256) area[i] = 0;
+}
+
 // Bit rows of CSR lists: bit x of row v (rw words, graph-relative ids) is set when x is in
 // v's list. Bound by reading the lists once and writing the rows once: one workgroup per
 // row gathers it in LDS and writes it out whole. A list that is not strictly ascending,
-// leaves its graph's id range or (no_self) holds the vertex itself raises *bad: no bit row
-// then says the same as the list.
+// leaves its graph's id range or (out- and in-lists) holds the vertex itself raises *bad: no
+// bit row then says the same as the list.
 constexpr int ROW_TILE = 8192;  // words of a row gathered at a time (262,144 ids)
-__global__ __launch_bounds__(256) void bit_rows_kernel(const unsigned long long* __restrict__ off,
-                                                       const int32_t* __restrict__ nbr, int n,
-                                                       const int32_t* __restrict__ gbase, int ngraphs, int rw,
-                                                       bool no_self, uint32_t* __restrict__ rows, uint32_t* bad) {
+struct RowLists {  // two-hop, out, in
+    const unsigned long long* off[3];
+    const int32_t* nbr[3];
+};
+__global__ __launch_bounds__(256) void bit_rows_kernel(RowLists lists, int n, const int32_t* __restrict__ gbase, int ngraphs,
+                                                       int rw, uint32_t* __restrict__ rows, uint32_t* bad) {
     __shared__ uint32_t tile[ROW_TILE];
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, which = blockIdx.y;
+    const unsigned long long* __restrict__ off = lists.off[which];
+    const int32_t* __restrict__ nbr = lists.nbr[which];
+    const bool no_self = which > 0;
+    rows += (unsigned long long)which * (unsigned long long)n * (unsigned long long)rw;
     for (int v = blockIdx.x; v < n; v += gridDim.x) {
         int gb = 0;
         if (gbase) {  // the last graph that starts at or before v
@@ -3151,7 +3786,7 @@ dqc_status dqc_open(const dqc_config* cfg, dqc_handle** out) {
                 "occupancy"))
         return DQC_E_HIP;
     h->split_wg = cus * std::max(per_cu_s, 1);
-    if (!c.pool_tasks) c.pool_tasks = 32ull * (unsigned long long)h->workgroups;
+    if (!c.pool_tasks) c.pool_tasks = 64ull * (unsigned long long)h->workgroups;
     // non-blocking stream: every host read of its results synchronizes on it explicitly
     if (!hip_ok(h, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking), "hipStreamCreate")) return DQC_E_HIP;
     if (!hip_ok(h, hipEventCreate(&h->ev0), "hipEventCreate")) return DQC_E_HIP;
@@ -3236,11 +3871,13 @@ static unsigned long long scratch_slots(const dqc_handle* h) {
 }
 
 // Zeroes the bitmaps of every workgroup's scratch area (the id-indexed values and lists
-// before them are written before they are read).
+// before them are written before they are read). Graphs all of whose tasks run on the
+// wavefront kernel use none (its bitmaps are in LDS, and it plans no chunks).
 static bool clear_bitmaps(dqc_handle* h, const char* what) {
-    const size_t pitch = sizeof(uint32_t) * h->stride, at = sizeof(uint32_t) * 22ull * (size_t)h->kloc;
-    return hip_ok(h, hipMemset2D((char*)h->d_scratch + at, pitch, 0, sizeof(uint32_t) * (size_t)h->bitmap_words(),
-                                 (size_t)scratch_slots(h) + 1), what);
+    if (wave_resident(h)) return true;
+    clear_kernel<<<(unsigned)(scratch_slots(h) + 1), 256, 0, h->stream>>>(h->d_scratch, h->stride,
+                                                                          22ull * (unsigned long long)h->kloc);
+    return hip_ok(h, hipGetLastError(), what) && hip_ok(h, hipStreamSynchronize(h->stream), what);
 }
 
 // Most memory the three sets of bit rows may take: 16 GiB, graphs of up to 214,000
@@ -3249,12 +3886,11 @@ constexpr unsigned long long MAX_ROW_BYTES = 16ull << 30;
 
 // Bit rows of the uploaded graph's lists. Graphs whose rows would exceed MAX_ROW_BYTES (or
 // the free memory), and lists that are not strictly ascending, keep none: the kernels then
-// walk the lists. Neither do graphs all of whose tasks the wavefront kernel runs, which
-// walks lists (building rows made opening a 1,000-vertex graph 1.6 ms longer).
+// walk the lists.
 static dqc_status build_rows(dqc_handle* h) {
     h->rw = ((h->kloc + 31) / 32 + 3) & ~3;
     const unsigned long long words = (unsigned long long)h->n * (unsigned long long)h->rw;
-    if (h->n == 0 || wave_resident(h) || 3 * words * sizeof(uint32_t) > MAX_ROW_BYTES) return DQC_OK;
+    if (h->n == 0 || 3 * words * sizeof(uint32_t) > MAX_ROW_BYTES) return DQC_OK;
     void* q = nullptr;
     if (hipMalloc(&q, (3 * words + 1) * sizeof(uint32_t)) != hipSuccess) {
         (void)hipGetLastError();
@@ -3263,13 +3899,10 @@ static dqc_status build_rows(dqc_handle* h) {
     h->allocs.push_back(q);
     h->d_rows = (uint32_t*)q;
     uint32_t bad = 0, *d_bad = h->d_rows + 3 * words;
-    if (!hip_ok(h, hipMemcpy(d_bad, &bad, sizeof bad, hipMemcpyHostToDevice), "bit rows")) return DQC_E_HIP;
-    const int32_t* gb = h->ngraphs > 1 ? h->d_gbase : nullptr;
-    const int grid = std::min(h->n, 8192);
-    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_to, h->d_tn, h->n, gb, h->ngraphs, h->rw, false, h->d_rows, d_bad);
-    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_oo, h->d_on, h->n, gb, h->ngraphs, h->rw, true, h->d_rows + words, d_bad);
-    bit_rows_kernel<<<grid, 256, 0, h->stream>>>(h->d_io, h->d_in, h->n, gb, h->ngraphs, h->rw, true, h->d_rows + 2 * words,
-                                                 d_bad);
+    if (!hip_ok(h, hipMemsetAsync(d_bad, 0, sizeof bad, h->stream), "bit rows")) return DQC_E_HIP;
+    const RowLists lists{{h->d_to, h->d_oo, h->d_io}, {h->d_tn, h->d_on, h->d_in}};
+    bit_rows_kernel<<<dim3(std::min(h->n, 8192), 3), 256, 0, h->stream>>>(lists, h->n, h->ngraphs > 1 ? h->d_gbase : nullptr,
+                                                                         h->ngraphs, h->rw, h->d_rows, d_bad);
     if (!hip_ok(h, hipGetLastError(), "bit rows launch") ||
         !hip_ok(h, hipMemcpyAsync(&bad, d_bad, sizeof bad, hipMemcpyDeviceToHost, h->stream), "bit rows") ||
         !hip_ok(h, hipStreamSynchronize(h->stream), "bit rows"))
@@ -3755,7 +4388,9 @@ static KParams make_params(dqc_handle* h, unsigned long long ntask) {
     P.b2 = h->d_rows;
     P.bo = h->d_rows ? h->d_rows + words : nullptr;
     P.bi = h->d_rows ? h->d_rows + 2 * words : nullptr;
+    P.rows_bad = nullptr;
     P.rw = h->rw;
+    P.tlen = h->tlen;
     P.max_depth = (uint32_t)std::max(0, h->cfg.max_depth);
     P.root_steps = std::max(0, h->cfg.root_branches);
     P.root_first = std::max(0, h->cfg.root_first);

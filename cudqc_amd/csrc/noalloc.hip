@@ -13,11 +13,15 @@ namespace {
 
 constexpr int NOALLOC_KMAX = 4096;  // largest condensed graph (vertices)
 constexpr int NOALLOC_WG = 256;     // workgroups per launch (one per CU)
-constexpr unsigned long long NOALLOC_STRIDE = 22ull * NOALLOC_KMAX;  // uint32 words per workgroup (even)
-constexpr unsigned long long NOALLOC_CTR_WORDS = 256;                // QCtr + GCtr, padded
-constexpr unsigned long long NOALLOC_WORDS = NOALLOC_CTR_WORDS + NOALLOC_STRIDE * NOALLOC_WG;
-static_assert(sizeof(QCtr) + sizeof(GCtr) <= NOALLOC_CTR_WORDS * 4, "counter area");
-static_assert(NOALLOC_STRIDE % 2 == 0, "8-byte aligned workgroup areas");
+constexpr int NOALLOC_RW = NOALLOC_KMAX / 32;  // words of a bit row
+// uint32 words per workgroup: the id-indexed values and lists, then the chunk planner's
+// bitmaps at the end (all-zero between tasks, whatever the graph's size)
+constexpr unsigned long long NOALLOC_STRIDE = 22ull * NOALLOC_KMAX + CHUNK_WORDS * NOALLOC_RW;
+constexpr unsigned long long NOALLOC_CTR_WORDS = 1024;  // QCtr + GCtr, padded; the last word: RowLists' bad flag
+constexpr unsigned long long NOALLOC_ROW_WORDS = 3ull * NOALLOC_KMAX * NOALLOC_RW;
+constexpr unsigned long long NOALLOC_WORDS = NOALLOC_CTR_WORDS + NOALLOC_STRIDE * NOALLOC_WG + NOALLOC_ROW_WORDS;
+static_assert(sizeof(QCtr) + sizeof(GCtr) + 256 + 4 <= NOALLOC_CTR_WORDS * 4, "counter area");
+static_assert(NOALLOC_STRIDE % 4 == 0, "16-byte aligned workgroup areas");
 
 // The scratch array. In host code `scratch` names a host-side stand-in, never device
 // memory: host code uses only the per-device address obtained from
@@ -46,14 +50,16 @@ hipError_t noalloc_scratch(uint32_t** out) {
 }
 
 // Sets the launch counters for a batch of `ntask` tasks and `nrec` records (every field
-// the expansion reads; nothing is left from an earlier call). One thread.
-__global__ void noalloc_init_kernel(QCtr* q, GCtr* g, unsigned long long ntask, unsigned long long nrec) {
-    QCtr qc{};
-    qc.root_first = ~0ull;
-    qc.ntask = ntask;
-    qc.pend = (ntask << CNT_SHIFT) | nrec;
-    *q = qc;
-    *g = GCtr{};
+// the expansion reads; nothing is left from an earlier call). One workgroup; ctr is the
+// counter area.
+__global__ void noalloc_init_kernel(uint32_t* ctr, QCtr* q, unsigned long long ntask, unsigned long long nrec) {
+    for (int i = threadIdx.x; i < (int)NOALLOC_CTR_WORDS; i += blockDim.x) ctr[i] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        q->root_first = ~0ull;
+        q->ntask = ntask;
+        q->pend = (ntask << CNT_SHIFT) | nrec;
+    }
 }
 
 // Copies the outcome into the caller's counters (DQC_NOALLOC_COUNTERS entries).
@@ -109,7 +115,8 @@ extern "C" dqc_status dqc_expand_noalloc(const dqc_device_graph* graph, const dq
     hipStream_t s = (hipStream_t)stream;
     QCtr* q = (QCtr*)base;
     GCtr* g = (GCtr*)((char*)base + ((sizeof(QCtr) + 255) / 256) * 256);
-    noalloc_init_kernel<<<1, 1, 0, s>>>(q, g, (unsigned long long)ntasks, (unsigned long long)nrecords);
+    uint32_t* bad = base + NOALLOC_CTR_WORDS - 1;
+    noalloc_init_kernel<<<1, 256, 0, s>>>(base, q, (unsigned long long)ntasks, (unsigned long long)nrecords);
     if (ntasks > 0) {
         KParams P{};
         P.n = graph->n;
@@ -147,8 +154,25 @@ extern "C" dqc_status dqc_expand_noalloc(const dqc_device_graph* graph, const dq
         P.root_steps = 0;
         P.maxtot = (unsigned long long)std::max(max_task_size, 1);
         P.gbase = nullptr;
+        // bit rows of the caller's lists: one small launch, 6 to 50 us for 100 to 4,096
+        // vertices, against 50 us a step of a task that has to walk lists
+        uint32_t* rows = base + NOALLOC_CTR_WORDS + NOALLOC_STRIDE * NOALLOC_WG;
+        P.rw = ((graph->n + 31) / 32 + 3) & ~3;
+        const unsigned long long words = (unsigned long long)graph->n * (unsigned long long)P.rw;
+        P.b2 = rows; P.bo = rows + words; P.bi = rows + 2 * words;
+        P.rows_bad = bad;
+        P.tlen = graph->table_len;
+        const RowLists lists{{P.to, P.oo, P.io}, {P.tn, P.on, P.in}};
+        if (graph->n > 0)
+            bit_rows_kernel<<<dim3(graph->n, 3), 256, 0, s>>>(lists, graph->n, nullptr, 1, P.rw, rows, bad);
         const int grid = (int)std::min<int64_t>(NOALLOC_WG, ntasks);
-        expand_kernel<false><<<grid, NT, 0, s>>>(P);
+        // tasks that fit a wavefront's lanes run on single wavefronts (a 24-vertex task of 7
+        // branches: 211 us a call, 428 us on a workgroup that walks lists); the grid is the same,
+        // and with it the stack margin
+        if (graph->n <= WAVE_KMAX && max_task_size <= LANE_TASK)
+            expand_kernel<false, WAVE_T, WAVE_KW><<<grid, WAVE_T, 0, s>>>(P);
+        else
+            expand_kernel<false><<<grid, NT, 0, s>>>(P);
     }
     noalloc_finish_kernel<<<1, 1, 0, s>>>(q, g, (unsigned long long*)counters);
     return hipGetLastError() == hipSuccess ? DQC_OK : DQC_E_HIP;

@@ -33,7 +33,7 @@ typedef struct dqc_handle dqc_handle;
 typedef struct {
     int32_t device;            /* HIP device ordinal                                  */
     int32_t workgroups;        /* persistent workgroups; 0 = as many as are resident  */
-    uint64_t pool_tasks;       /* tasks expanded per launch (batch); 0 = 32 per WG    */
+    uint64_t pool_tasks;       /* tasks expanded per launch (batch); 0 = 64 per WG    */
     uint64_t pool_vertices;    /* 24-byte vertex records the batch buffer holds       */
     uint64_t spill_tasks;      /* task descriptors the LIFO task stack holds          */
     uint64_t spill_vertices;   /* vertex records the LIFO task stack holds            */

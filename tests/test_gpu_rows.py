@@ -1,8 +1,7 @@
-"""Planned steps on bit rows (the workgroup kernels) against the oracle at the sizes where
-words, chunks and planes end: condensed graphs of 31 to 129 vertices (32 ids a word), tasks of
+"""Planned steps on bit rows (the workgroup kernels) and tasks with a vertex per lane (the
+wavefront kernel) against the oracle at the sizes where words, chunks, planes and lanes end: condensed graphs of 31 to 129 vertices (32 ids a word), tasks of
 one to a few chunks of 32 steps, member counts beyond the bit planes (14) and least clique
-sizes on either side of them. The wavefront kernel walks lists instead, so it is run on the
-same graphs as a second reference. Also: lists that no bit row can stand for are walked."""
+sizes on either side of them. Also: lists that no bit row can stand for are walked."""
 import ctypes
 import os
 import random
@@ -65,6 +64,17 @@ def test_planned_steps_match_oracle(dqc, tmp_path, case):
         data = open(got_path, "rb").read() if os.path.exists(got_path) else b""
         assert (got, gst.tasks_expanded, gst.branches, gst.raw_cliques) == (count, st.tasks, st.branches, st.raw_cliques)
         assert data == want
+    # two copies in one batch: the level-0 tasks (31 to 129 vertices, on either side of the 64
+    # lanes) run as ordinary tasks, small ones with a vertex per lane, their results buffered
+    for resident in (0, 3):
+        cfg = dqc.Config()
+        cfg.host_addfail_check = 1
+        cfg.resident_steps = resident
+        files = [str(tmp_path / f"batch{resident}_{i}.max") for i in range(2)]
+        counts, bst = dqc.search_batch([path, path], go, gi, mn, files, cfg)
+        assert counts == [count, count]
+        assert (bst.tasks_expanded, bst.branches, bst.raw_cliques) == (2 * st.tasks, 2 * st.branches, 2 * st.raw_cliques)
+        assert all((open(f, "rb").read() if os.path.exists(f) else b"") == want for f in files)
 
 
 def run_uploaded(dqc, lists, records, mn, gamma):
