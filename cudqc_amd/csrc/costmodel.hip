@@ -2,10 +2,9 @@
 // and their C-ABI (include/dqc.h). The model orders and splits the task batches of the
 // learned schedule; it changes only the order in which tasks run, never the output.
 //
-// Training is deterministic: each workgroup processes chunks of 64 samples through LDS
-// activation tiles, every thread accumulates the gradient of a fixed set of parameters
-// in registers, per-workgroup partial gradients are reduced in a fixed order, and Adam
-// applies the step.
+// Training is deterministic: each workgroup takes chunks of 64 samples through the network
+// on matrix cores, accumulates its weight gradients in registers, and the partial gradients
+// are summed in a fixed order by the kernel that applies the Adam step.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,154 +23,225 @@ using namespace dqc_cost;
 
 constexpr int GT = 256;                              // threads per training workgroup
 constexpr int CH = 64;                               // samples per chunk
-constexpr int OWN = (NPARAM + GT - 1) / GT;          // parameters owned per thread (19)
 constexpr int MAX_BLOCKS = 512;
 
 static_assert(NPARAM == DQC_MLP_PARAMS, "parameter count");
 static_assert(IN == DQC_MLP_IN && H == DQC_MLP_HIDDEN, "model shape");
 
+// The network on matrix cores in fp32 (v_mfma_f32_16x16x4: operand and result layout of the
+// CDNA ISA). A wavefront takes 16 samples: units are rows and samples columns, so lane l
+// holds sample l % 16 and, in register 4 t + r, unit 16 t + 4 (l / 16) + r. A layer's result has
+// the layout in which the next product takes it as its right operand, with the units summed
+// in the order (t, r), so activations never leave the registers between layers.
+typedef float f4 __attribute__((ext_vector_type(4)));
+constexpr int LDW = H + 1;  // row stride of a 64-wide LDS matrix (banks)
+struct Act { f4 v[4]; };     // 64 units x 16 samples
+__device__ __forceinline__ float relu(float z) { return z > 0.f ? z : 0.f; }
+__device__ __forceinline__ int unit_of(int t, int r, int lane) { return 16 * t + 4 * (lane >> 4) + r; }
+__device__ __forceinline__ Act unit_values(const float* p, int lane) {  // p[unit], for each of the lane's units
+    Act a;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a.v[t][r] = p[unit_of(t, r, lane)];
+    return a;
+}
+// acc[u] (rows 16 u ..) += A (64 x 64) * B, A's operand given by a(u, k) with k = 4 t + r standing
+// for column unit_of(t, r, lane) of row 16 u + lane % 16
+template <class F>
+__device__ __forceinline__ void mul64(Act& acc, const Act& B, F&& a) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                acc.v[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a(u, 4 * t + r), B.v[t][r], acc.v[u], 0, 0, 0);
+}
+// First layer before its ReLU: z = b1 + W1 x, the 7 features padded to 8. x0 / x1: features
+// lane / 16 and 4 + lane / 16 of the lane's sample.
+__device__ __forceinline__ Act layer1(const float* p, const Act& b1, float x0, float x1, int lane) {
+    Act z = b1;
+    const int k = lane >> 4;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const float* w = p + OFF_W1 + (16 * u + (lane & 15)) * IN;
+        z.v[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k], x0, z.v[u], 0, 0, 0);
+        z.v[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(k < 3 ? w[4 + k] : 0.f, x1, z.v[u], 0, 0, 0);
+    }
+    return z;
+}
+__device__ __forceinline__ Act relu(Act a) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a.v[t][r] = relu(a.v[t][r]);
+    return a;
+}
+// sum over the lane's units of w * b, then over the four lanes of its sample
+__device__ __forceinline__ float head(const Act& w, const Act& b, float b3) {
+    float y = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) y += w.v[t][r] * b.v[t][r];
+    y += __shfl_xor(y, 16, 64);
+    y += __shfl_xor(y, 32, 64);
+    return y + b3;
+}
+
+// y = the network's prediction for n samples. Bound by the fp32 matrix rate: 72 products of
+// 16x16x4 a wavefront per 16 samples; the second layer's weights stay in registers.
+// 262,144 samples: 37 us (one sample per thread, weights in LDS: 195 us).
 __global__ __launch_bounds__(256) void forward_kernel(const float* __restrict__ params, const float* __restrict__ x,
                                                       long long n, float* __restrict__ y) {
     __shared__ float p[NPARAM];
     for (int i = threadIdx.x; i < NPARAM; i += blockDim.x) p[i] = params[i];
     __syncthreads();
-    for (long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x; s < n; s += (long long)gridDim.x * blockDim.x)
-        y[s] = forward(p, x + IN * s);
+    const int lane = threadIdx.x & 63;
+    const Act b1 = unit_values(p + OFF_B1, lane), b2 = unit_values(p + OFF_B2, lane), w3 = unit_values(p + OFF_W3, lane);
+    float w2[4][16];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < 16; ++k)
+            w2[u][k] = p[OFF_W2 + (16 * u + (lane & 15)) * H + unit_of(k >> 2, k & 3, lane)];
+    const float b3 = p[OFF_B3];
+    const long long waves = (long long)gridDim.x * (blockDim.x >> 6);
+    for (long long s0 = ((long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 16; s0 < n; s0 += 16 * waves) {
+        const long long s = s0 + (lane & 15);
+        const int k = lane >> 4;
+        const float x0 = s < n ? x[IN * s + k] : 0.f, x1 = s < n && k < 3 ? x[IN * s + 4 + k] : 0.f;
+        const Act a = relu(layer1(p, b1, x0, x1, lane));
+        Act z = b2;
+        mul64(z, a, [&](int u, int k2) { return w2[u][k2]; });
+        const float v = head(w3, relu(z), b3);
+        if (lane < 16 && s < n) y[s] = v;
+    }
 }
 
 // Gradient of sum_s scale * (y_s - t_s)^2 over samples idx[0..m) (idx null: 0..m-1).
-// partial[block][p] gets the block's share, lpart[block] its sum of squared errors.
-__global__ __launch_bounds__(GT) void grad_kernel(const float* __restrict__ p, const float* __restrict__ x,
-                                                  const float* __restrict__ t, const int32_t* __restrict__ idx,
-                                                  long long m, float scale, float* __restrict__ partial,
-                                                  double* __restrict__ lpart) {
-    __shared__ float xs[CH][IN];
-    __shared__ float ts[CH];
-    __shared__ float dy[CH];
-    __shared__ float A[CH][H];   // first hidden layer (after ReLU)
-    __shared__ float B[CH][H];   // second hidden layer, then its pre-activation gradient
-    __shared__ float C[CH][H];   // pre-activation gradient of the first hidden layer
+// partial[block][p] gets the block's share, lpart[block] its sum of squared errors (GRAD
+// false: only that). Each of the four wavefronts takes 16 samples of a chunk through both
+// passes in registers; the weight gradients are products over the chunk's 64 samples, whose
+// activations and pre-activation gradients meet in LDS, and stay in accumulators over the
+// block's chunks. Bound by latency at a training batch (1,024 samples are 16 workgroups of one
+// chunk): 17 us a call there, 58 us with vector instructions.
+template <bool GRAD>
+__global__ __launch_bounds__(GT, 1) void grad_kernel(const float* __restrict__ params, const float* __restrict__ x,
+                                                     const float* __restrict__ t, const int32_t* __restrict__ idx,
+                                                     long long m, float scale, float* __restrict__ partial,
+                                                     double* __restrict__ lpart) {
+    __shared__ float p[NPARAM];
+    __shared__ float A[H * LDW];  // [unit][sample]: first hidden layer
+    __shared__ float B[H * LDW];  // pre-activation gradient of the second hidden layer
+    __shared__ float C[H * LDW];  // and of the first
+    __shared__ float X[8 * LDW];  // [feature][sample], feature 7 = 1 (the bias)
     __shared__ double lred[GT];
-    const int tid = threadIdx.x;
-    float acc[OWN];
-#pragma unroll
-    for (int k = 0; k < OWN; ++k) acc[k] = 0.f;
+    __shared__ float red[2][4][H];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, k = lane >> 4;
+    for (int i = tid; i < NPARAM; i += GT) p[i] = params[i];
+    __syncthreads();
+    const Act b1 = unit_values(p + OFF_B1, lane), b2 = unit_values(p + OFF_B2, lane), w3 = unit_values(p + OFF_W3, lane);
+    const float b3 = p[OFF_B3];
+    f4 g2[4] = {}, g1 = {};   // this wavefront's rows 16 wave .. of dW2 (4 column tiles) and of dW1 | db1
+    Act gw3 = {}, gb2 = {};
+    float gb3 = 0.f;
     double loss = 0.0;
     const long long nchunk = (m + CH - 1) / CH;
     for (long long c = blockIdx.x; c < nchunk; c += gridDim.x) {
-        const long long base = c * CH;
-        const int cnt = (int)std::min<long long>(CH, m - base);
-        for (int e = tid; e < CH * IN; e += GT) {
-            const int s = e / IN, f = e % IN;
-            float v = 0.f;
-            if (s < cnt) {
-                const long long g = idx ? (long long)idx[base + s] : base + s;
-                v = x[g * IN + f];
-            }
-            xs[s][f] = v;
-        }
-        if (tid < CH) {
-            float v = 0.f;
-            if (tid < cnt) v = t[idx ? (long long)idx[base + tid] : base + tid];
-            ts[tid] = v;
-        }
-        __syncthreads();
-        for (int e = tid; e < CH * H; e += GT) {  // layer 1
-            const int s = e / H, j = e % H;
-            float z = p[OFF_B1 + j];
+        const long long s = c * CH + 16 * wave + col;
+        const bool live = s < m;
+        const long long at = live ? (idx ? (long long)idx[s] : s) : 0;
+        const float x0 = live ? x[at * IN + k] : 0.f, x1 = live && k < 3 ? x[at * IN + 4 + k] : 0.f;
+        const Act a = relu(layer1(p, b1, x0, x1, lane));
+        Act z = b2;
+        mul64(z, a, [&](int u, int kk) { return p[OFF_W2 + (16 * u + col) * H + unit_of(kk >> 2, kk & 3, lane)]; });
+        const Act b = relu(z);
+        const float r = live ? head(w3, b, b3) - t[at] : 0.f;
+        if (lane < 16) loss += (double)r * (double)r;
+        if (!GRAD) continue;
+        const float dy = 2.f * scale * r;
+        if (lane < 16) gb3 += dy;
+        Act db;
 #pragma unroll
-            for (int f = 0; f < IN; ++f) z += p[OFF_W1 + j * IN + f] * xs[s][f];
-            A[s][j] = z > 0.f ? z : 0.f;
-        }
-        __syncthreads();
-        for (int e = tid; e < CH * H; e += GT) {  // layer 2
-            const int s = e / H, j = e % H;
-            float z = p[OFF_B2 + j];
-            for (int i = 0; i < H; ++i) z += p[OFF_W2 + j * H + i] * A[s][i];
-            B[s][j] = z > 0.f ? z : 0.f;
-        }
-        __syncthreads();
-        if (tid < CH) {  // output, loss and its gradient
-            float y = p[OFF_B3];
-            for (int j = 0; j < H; ++j) y += p[OFF_W3 + j] * B[tid][j];
-            const float r = tid < cnt ? y - ts[tid] : 0.f;
-            dy[tid] = 2.f * scale * r;
-            loss += (double)r * (double)r;
-        }
-        __syncthreads();
-        // dW3, db3 (B still holds the second hidden layer)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int k = 0; k < OWN; ++k) {
-            const int q = tid + k * GT;
-            if (q >= OFF_W3 && q < NPARAM) {
-                float g = 0.f;
-                if (q == OFF_B3) {
-                    for (int s = 0; s < CH; ++s) g += dy[s];
-                } else {
-                    const int j = q - OFF_W3;
-                    for (int s = 0; s < CH; ++s) g += dy[s] * B[s][j];
-                }
-                acc[k] += g;
+            for (int e = 0; e < 4; ++e) {
+                gw3.v[q][e] += dy * b.v[q][e];
+                db.v[q][e] = b.v[q][e] > 0.f ? dy * w3.v[q][e] : 0.f;
+                gb2.v[q][e] += db.v[q][e];
             }
-        }
-        __syncthreads();
-        for (int e = tid; e < CH * H; e += GT) {
-            const int s = e / H, j = e % H;
-            B[s][j] = B[s][j] > 0.f ? dy[s] * p[OFF_W3 + j] : 0.f;
-        }
-        __syncthreads();
-        // dW2, db2
+        Act da = {};
+        mul64(da, db, [&](int u, int kk) { return p[OFF_W2 + unit_of(kk >> 2, kk & 3, lane) * H + 16 * u + col]; });
+        __syncthreads();  // (the previous chunk's products are done with the LDS matrices)
+        const int sc = 16 * wave + col;
 #pragma unroll
-        for (int k = 0; k < OWN; ++k) {
-            const int q = tid + k * GT;
-            if (q >= OFF_W2 && q < OFF_W3) {
-                float g = 0.f;
-                if (q >= OFF_B2) {
-                    const int j = q - OFF_B2;
-                    for (int s = 0; s < CH; ++s) g += B[s][j];
-                } else {
-                    const int j = (q - OFF_W2) / H, i = (q - OFF_W2) % H;
-                    for (int s = 0; s < CH; ++s) g += B[s][j] * A[s][i];
-                }
-                acc[k] += g;
-            }
-        }
-        for (int e = tid; e < CH * H; e += GT) {
-            const int s = e / H, i = e % H;
-            float g = 0.f;
-            if (A[s][i] > 0.f)
-                for (int j = 0; j < H; ++j) g += B[s][j] * p[OFF_W2 + j * H + i];
-            C[s][i] = g;
-        }
-        __syncthreads();
-        // dW1, db1
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int k = 0; k < OWN; ++k) {
-            const int q = tid + k * GT;
-            if (q < OFF_W2) {
-                float g = 0.f;
-                if (q >= OFF_B1) {
-                    const int j = q - OFF_B1;
-                    for (int s = 0; s < CH; ++s) g += C[s][j];
-                } else {
-                    const int j = q / IN, f = q % IN;
-                    for (int s = 0; s < CH; ++s) g += C[s][j] * xs[s][f];
-                }
-                acc[k] += g;
+            for (int e = 0; e < 4; ++e) {
+                const int u = unit_of(q, e, lane);
+                A[u * LDW + sc] = a.v[q][e];
+                B[u * LDW + sc] = db.v[q][e];
+                C[u * LDW + sc] = a.v[q][e] > 0.f ? da.v[q][e] : 0.f;
             }
-        }
+        X[k * LDW + sc] = x0;
+        X[(4 + k) * LDW + sc] = k < 3 ? x1 : live ? 1.f : 0.f;
         __syncthreads();
+        const int row = 16 * wave + col;
+#pragma unroll 4
+        for (int kb = 0; kb < CH / 4; ++kb) {
+            const int ss = 4 * kb + k;
+            const float fb = B[row * LDW + ss], fc = C[row * LDW + ss];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                g2[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb, A[(16 * u + col) * LDW + ss], g2[u], 0, 0, 0);
+            g1 = __builtin_amdgcn_mfma_f32_16x16x4f32(fc, col < 8 ? X[col * LDW + ss] : 0.f, g1, 0, 0, 0);
+        }
     }
+    if (GRAD) {
+        float* out = partial + (long long)blockIdx.x * NPARAM;
 #pragma unroll
-    for (int k = 0; k < OWN; ++k) {
-        const int q = tid + k * GT;
-        if (q < NPARAM) partial[(long long)blockIdx.x * NPARAM + q] = acc[k];
+        for (int e = 0; e < 4; ++e) {
+            const int j = 16 * wave + 4 * k + e;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) out[OFF_W2 + j * H + 16 * u + col] = g2[u][e];
+            if (col < IN) out[OFF_W1 + j * IN + col] = g1[e];
+            else if (col == IN) out[OFF_B1 + j] = g1[e];
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float w = gw3.v[q][e], v = gb2.v[q][e];
+                for (int off = 8; off > 0; off >>= 1) {  // over the wavefront's 16 samples
+                    w += __shfl_xor(w, off, 64);
+                    v += __shfl_xor(v, off, 64);
+                }
+                if (col == 0) {
+                    red[0][wave][unit_of(q, e, lane)] = w;
+                    red[1][wave][unit_of(q, e, lane)] = v;
+                }
+            }
+        for (int off = 8; off > 0; off >>= 1) gb3 += __shfl_xor(gb3, off, 64);
     }
     lred[tid] = loss;
     __syncthreads();
+    if (GRAD) {
+        float* out = partial + (long long)blockIdx.x * NPARAM;
+        if (tid < 2 * H) {
+            const int q = tid / H, j = tid % H;
+            out[(q ? OFF_B2 : OFF_W3) + j] = red[q][0][j] + red[q][1][j] + red[q][2][j] + red[q][3][j];
+        }
+        __syncthreads();
+        if (lane == 0) red[0][wave][0] = gb3;
+        __syncthreads();
+        if (tid == 0) out[OFF_B3] = red[0][0][0] + red[0][1][0] + red[0][2][0] + red[0][3][0];
+    }
     if (tid == 0) {
         double sum = 0.0;
-        for (int i = 0; i < GT; ++i) sum += lred[i];
+        for (int w = 0; w < 4; ++w)
+            for (int i = 0; i < 16; ++i) sum += lred[64 * w + i];  // (a sample's error is in its first lane)
         lpart[blockIdx.x] = sum;
     }
 }
@@ -185,13 +255,18 @@ __global__ void reduce_kernel(const float* __restrict__ partial, int nblocks, fl
     grad[q] = g;
 }
 
-__global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ mo,
+// One Adam step on the blocks' partial gradients (summed in block order, as reduce_kernel
+// does): one launch instead of two, bound by its latency.
+__global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ partial, int nblocks, float* __restrict__ mo,
                             float* __restrict__ ve, float lr, float c1, float c2) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= NPARAM) return;
+    float g = 0.f;
+#pragma unroll 8
+    for (int b = 0; b < nblocks; ++b) g += partial[(long long)b * NPARAM + q];
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float m = b1 * mo[q] + (1.f - b1) * g[q];
-    const float v = b2 * ve[q] + (1.f - b2) * g[q] * g[q];
+    const float m = b1 * mo[q] + (1.f - b1) * g;
+    const float v = b2 * ve[q] + (1.f - b2) * g * g;
     mo[q] = m;
     ve[q] = v;
     p[q] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
@@ -216,12 +291,17 @@ int grad_blocks(long long m) {
     return (int)std::max<long long>(1, std::min<long long>(MAX_BLOCKS, (m + CH - 1) / CH));
 }
 
-// Full-data gradient on device buffers; returns the sum of squared errors.
+// Full-data gradient (dgrad null: only the error) on device buffers; gives the sum of squared
+// errors.
 bool device_gradient(const float* dp, const float* dx, const float* dt, long long n, float* dgrad, float* dpart,
                      double* dl, double* sse) {
     const int nb = grad_blocks(n);
-    grad_kernel<<<nb, GT>>>(dp, dx, dt, nullptr, n, 1.f / (float)n, dpart, dl);
-    reduce_kernel<<<(NPARAM + 255) / 256, 256>>>(dpart, nb, dgrad);
+    if (dgrad) {
+        grad_kernel<true><<<nb, GT>>>(dp, dx, dt, nullptr, n, 1.f / (float)n, dpart, dl);
+        reduce_kernel<<<(NPARAM + 255) / 256, 256>>>(dpart, nb, dgrad);
+    } else {
+        grad_kernel<false><<<nb, GT>>>(dp, dx, dt, nullptr, n, 1.f / (float)n, dpart, dl);
+    }
     std::vector<double> l(nb);
     if (hipMemcpy(l.data(), dl, sizeof(double) * nb, hipMemcpyDeviceToHost) != hipSuccess) return false;
     double s = 0.0;
@@ -250,7 +330,7 @@ dqc_status dqc_mlp_forward(const float* params, const float* x, int64_t n, float
     if (hipMemcpy(dp, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dx, x, sizeof(float) * IN * (size_t)n, hipMemcpyHostToDevice) != hipSuccess)
         return DQC_E_HIP;
-    const int blocks = (int)std::min<long long>(4096, (n + 255) / 256);
+    const int blocks = (int)std::min<long long>(768, (n + 63) / 64);  // three workgroups a CU, 16 samples a wavefront
     forward_kernel<<<blocks, 256>>>(dp, dx, n, dy);
     if (hipGetLastError() != hipSuccess ||
         hipMemcpy(y, dy, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost) != hipSuccess)
@@ -285,11 +365,11 @@ dqc_status dqc_mlp_train(float* params, const float* x, const float* t, int64_t 
     const int nb = grad_blocks(std::min<long long>(n, batch));
     const int nbf = grad_blocks(n);
     float *dp = b.alloc<float>(NPARAM), *dx = b.alloc<float>((size_t)n * IN), *dt = b.alloc<float>((size_t)n);
-    float *dg = b.alloc<float>(NPARAM), *dm = b.alloc<float>(NPARAM), *dv = b.alloc<float>(NPARAM);
-    float* dpart = b.alloc<float>((size_t)std::max(nb, nbf) * NPARAM);
+    float *dm = b.alloc<float>(NPARAM), *dv = b.alloc<float>(NPARAM);
+    float* dpart = b.alloc<float>((size_t)nb * NPARAM);
     double* dl = b.alloc<double>(std::max(nb, nbf));
     int32_t* didx = b.alloc<int32_t>((size_t)n);
-    if (!dp || !dx || !dt || !dg || !dm || !dv || !dpart || !dl || !didx) return DQC_E_HIP;
+    if (!dp || !dx || !dt || !dm || !dv || !dpart || !dl || !didx) return DQC_E_HIP;
     if (hipMemcpy(dp, params, sizeof(float) * NPARAM, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dx, x, sizeof(float) * IN * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dt, t, sizeof(float) * (size_t)n, hipMemcpyHostToDevice) != hipSuccess ||
@@ -309,16 +389,15 @@ dqc_status dqc_mlp_train(float* params, const float* x, const float* t, int64_t 
         for (long long s0 = 0; s0 < n; s0 += batch) {
             const long long m = std::min<long long>(batch, n - s0);
             const int blocks = grad_blocks(m);
-            grad_kernel<<<blocks, GT>>>(dp, dx, dt, didx + s0, m, 1.f / (float)m, dpart, dl);
-            reduce_kernel<<<(NPARAM + 255) / 256, 256>>>(dpart, blocks, dg);
+            grad_kernel<true><<<blocks, GT>>>(dp, dx, dt, didx + s0, m, 1.f / (float)m, dpart, dl);
             ++step;
             const float c1 = 1.f - powf(0.9f, (float)step), c2 = 1.f - powf(0.999f, (float)step);
-            adam_kernel<<<(NPARAM + 255) / 256, 256>>>(dp, dg, dm, dv, lr, c1, c2);
+            adam_kernel<<<(NPARAM + 63) / 64, 64>>>(dp, dpart, blocks, dm, dv, lr, c1, c2);
         }
         if (hipGetLastError() != hipSuccess) return DQC_E_HIP;
     }
     double sse = 0.0;
-    if (!device_gradient(dp, dx, dt, n, dg, dpart, dl, &sse)) return DQC_E_HIP;
+    if (!device_gradient(dp, dx, dt, n, nullptr, dpart, dl, &sse)) return DQC_E_HIP;
     if (hipMemcpy(params, dp, sizeof(float) * NPARAM, hipMemcpyDeviceToHost) != hipSuccess) return DQC_E_HIP;
     if (loss) *loss = sse / (double)n;
     return DQC_OK;
