@@ -4830,3 +4830,5 @@ dqc_status dqc_get_stats(const dqc_handle* h, dqc_stats* st) {
 
 // the allocation-free entry point launches the kernels above
 #include "noalloc.hip"
+// the device pass before the maximal-set filter reads the handle's clique store
+#include "prefilter.hip"

@@ -16,6 +16,7 @@
 
 #include "../../include/dqc.h"
 #include "graph.hpp"
+#include "prefilter.hpp"
 
 namespace {
 
@@ -172,18 +173,24 @@ dqc_status search_impl(dqc::Graph& g, bool has_two, double go, double gi, int32_
         const double prep_ms = ms_since(t_start);
         s = dqc_run(h, DQC_SCHED_DEFAULT);
         if (s != DQC_OK) return fail(s);
-        int64_t count = 0, total = 0;
-        s = dqc_fetch_cliques(h, &count, &total, nullptr, nullptr);
-        if (s != DQC_OK) return fail(s);
-        std::vector<int32_t> sizes((size_t)count), ids((size_t)total);
-        s = dqc_fetch_cliques(h, &count, &total, sizes.data(), ids.data());
+        std::vector<int32_t> sizes, ids;
+        if (raw_path) {  // the raw file holds every clique
+            int64_t count = 0, total = 0;
+            s = dqc_fetch_cliques(h, &count, &total, nullptr, nullptr);
+            if (s != DQC_OK) return fail(s);
+            sizes.resize((size_t)count);
+            ids.resize((size_t)total);
+            s = dqc_fetch_cliques(h, &count, &total, sizes.data(), ids.data());
+        } else {
+            s = dqc::fetch_candidates(h, nullptr, sizes, ids);
+        }
         if (s != DQC_OK) return fail(s);
         dqc_get_stats(h, &stats);
         dqc_close(h);
         stats.preprocess_ms = prep_ms;
-        sets.reserve((size_t)count);
+        sets.reserve(sizes.size());
         size_t q = 0;
-        for (int64_t i = 0; i < count; ++i) {
+        for (size_t i = 0; i < sizes.size(); ++i) {
             sets.emplace_back(ids.begin() + q, ids.begin() + q + sizes[i]);
             q += (size_t)sizes[i];
         }
@@ -382,11 +389,8 @@ dqc_status dqc_prepare_batch(dqc_handle* h, const char* const* graph_paths, int3
 
 dqc_status dqc_finish_batch(dqc_handle* h, const char* const* max_paths, int64_t* max_cliques, dqc_stats* st) {
     if (!h) return DQC_E_ARG;
-    int64_t count = 0, total = 0;
-    dqc_status s = dqc_fetch_batch_cliques(h, &count, &total, nullptr, nullptr, nullptr);
-    if (s != DQC_OK) return s;
-    std::vector<int32_t> gid((size_t)count), sizes((size_t)count), ids((size_t)total);
-    s = dqc_fetch_batch_cliques(h, &count, &total, gid.data(), sizes.data(), ids.data());
+    std::vector<int32_t> gid, sizes, ids;
+    dqc_status s = dqc::fetch_candidates(h, &gid, sizes, ids);
     if (s != DQC_OK) return s;
     dqc_stats stats{};
     dqc_get_stats(h, &stats);
@@ -395,7 +399,7 @@ dqc_status dqc_finish_batch(dqc_handle* h, const char* const* max_paths, int64_t
     if (s != DQC_OK) return s;
     std::vector<std::vector<std::vector<int32_t>>> sets((size_t)ngraphs);
     size_t p = 0;
-    for (int64_t c = 0; c < count; ++c) {
+    for (size_t c = 0; c < sizes.size(); ++c) {
         if (gid[c] < 0 || gid[c] >= ngraphs) return DQC_E_ARG;
         sets[gid[c]].emplace_back(ids.begin() + p, ids.begin() + p + sizes[c]);
         p += (size_t)sizes[c];
