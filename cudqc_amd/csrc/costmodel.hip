@@ -16,6 +16,7 @@
 
 #include "../../include/dqc.h"
 #include "costmodel.hpp"
+#include "devpool.hpp"
 
 namespace {
 
@@ -272,17 +273,19 @@ __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ par
     p[q] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
 }
 
-// Device buffers of one call; freed on scope exit.
+// Device buffers of one call; given back on scope exit, when nothing queued uses them.
 struct Buf {
-    std::vector<void*> ptrs;
+    std::vector<std::pair<void*, size_t>> ptrs;
     ~Buf() {
-        for (void* q : ptrs) hipFree(q);
+        if (!ptrs.empty()) hipStreamSynchronize(nullptr);
+        for (auto& q : ptrs) dqc::DevicePool::get().give(q.first, q.second);
     }
     template <class T>
     T* alloc(size_t count) {
         void* q = nullptr;
-        if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return nullptr;
-        ptrs.push_back(q);
+        const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+        if (dqc::DevicePool::get().take(&q, bytes) != hipSuccess) return nullptr;
+        ptrs.push_back({q, bytes});
         return (T*)q;
     }
 };

@@ -39,6 +39,7 @@
 
 #include "../../include/dqc.h"
 #include "costmodel.hpp"
+#include "devpool.hpp"
 #include "graph.hpp"
 
 namespace {
@@ -3665,7 +3666,7 @@ struct dqc_handle {
     float* d_model = nullptr;      // cost model (dqc_set_cost_model)
     float* d_cost = nullptr;       // per-task predictions of the current batch
     std::vector<float> hpred;
-    std::vector<void*> allocs;
+    std::vector<std::pair<void*, size_t>> allocs;  // device buffers (DevicePool) and their bytes
     // batch buffer and task stack capacities left to the library (dqc_config field 0):
     // sized from the graph when it is uploaded
     bool auto_pool_v = false, auto_spill_t = false, auto_spill_v = false;
@@ -3683,10 +3684,22 @@ bool hip_ok(dqc_handle* h, hipError_t e, const char* what) {
 template <class T>
 bool dev_alloc(dqc_handle* h, T** p, size_t count, const char* what) {
     void* q = nullptr;
-    if (!hip_ok(h, hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)), what)) return false;
-    h->allocs.push_back(q);
+    const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
+    if (!hip_ok(h, dqc::DevicePool::get().take(&q, bytes), what)) return false;
+    h->allocs.push_back({q, bytes});
     *p = (T*)q;
     return true;
+}
+
+// Gives a buffer of the handle back to the pool; nothing queued uses it any more.
+void dev_free(dqc_handle* h, void* p) {
+    for (size_t i = 0; i < h->allocs.size(); ++i)
+        if (h->allocs[i].first == p) {
+            if (h->stream) hipStreamSynchronize(h->stream);
+            dqc::DevicePool::get().give(p, h->allocs[i].second);
+            h->allocs.erase(h->allocs.begin() + (std::ptrdiff_t)i);
+            return;
+        }
 }
 
 void drop_graphs(dqc_handle* h) {
@@ -3702,8 +3715,7 @@ void free_graph(dqc_handle* h) {
                   h->d_lto, h->d_ltn, h->d_flags, h->d_split, h->d_gbase, h->d_rows};
     for (void* p : gp)
         if (p) {
-            hipFree(p);
-            h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), p), h->allocs.end());
+            dev_free(h, p);
         }
     h->d_oo = h->d_io = h->d_to = nullptr;
     h->d_on = h->d_in = h->d_tn = nullptr;
@@ -3809,7 +3821,7 @@ dqc_status dqc_close(dqc_handle* h) {
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
     drop_graphs(h);
-    for (void* p : h->allocs) hipFree(p);
+    for (auto& a : h->allocs) dqc::DevicePool::get().give(a.first, a.second);
     if (h->ev0) hipEventDestroy(h->ev0);
     if (h->ev1) hipEventDestroy(h->ev1);
     if (h->stream) hipStreamDestroy(h->stream);
@@ -3838,8 +3850,7 @@ static dqc_status size_buffers(dqc_handle* h) {
     auto realloc_buf = [&](auto** p, unsigned long long& cap, unsigned long long want, const char* what) {
         if (*p && cap == want) return true;
         if (*p) {
-            hipFree(*p);
-            h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), (void*)*p), h->allocs.end());
+            dev_free(h, *p);
             *p = nullptr;
         }
         cap = 0;
@@ -3892,11 +3903,12 @@ static dqc_status build_rows(dqc_handle* h) {
     const unsigned long long words = (unsigned long long)h->n * (unsigned long long)h->rw;
     if (h->n == 0 || 3 * words * sizeof(uint32_t) > MAX_ROW_BYTES) return DQC_OK;
     void* q = nullptr;
-    if (hipMalloc(&q, (3 * words + 1) * sizeof(uint32_t)) != hipSuccess) {
+    const size_t bytes = (3 * words + 1) * sizeof(uint32_t);
+    if (dqc::DevicePool::get().take(&q, bytes) != hipSuccess) {
         (void)hipGetLastError();
         return DQC_OK;
     }
-    h->allocs.push_back(q);
+    h->allocs.push_back({q, bytes});
     h->d_rows = (uint32_t*)q;
     uint32_t bad = 0, *d_bad = h->d_rows + 3 * words;
     if (!hip_ok(h, hipMemsetAsync(d_bad, 0, sizeof bad, h->stream), "bit rows")) return DQC_E_HIP;
@@ -3908,8 +3920,7 @@ static dqc_status build_rows(dqc_handle* h) {
         !hip_ok(h, hipStreamSynchronize(h->stream), "bit rows"))
         return DQC_E_HIP;
     if (bad) {
-        hipFree(q);
-        h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), q), h->allocs.end());
+        dev_free(h, q);
         h->d_rows = nullptr;
     }
     return DQC_OK;
@@ -4041,8 +4052,7 @@ dqc_status dqc_set_tables(dqc_handle* h, const int32_t* md_out, const int32_t* m
     drop_graphs(h);
     if (h->d_mdo) {
         for (void* p : {(void*)h->d_mdo, (void*)h->d_mdi, (void*)h->d_ubo, (void*)h->d_ubi}) {
-            hipFree(p);
-            h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), p), h->allocs.end());
+            dev_free(h, p);
         }
     }
     if (!dev_alloc(h, &h->d_mdo, len, "table alloc") || !dev_alloc(h, &h->d_mdi, len, "table alloc") ||
@@ -4724,8 +4734,7 @@ dqc_status dqc_set_task_log(dqc_handle* h, int64_t capacity) {
     hipSetDevice(h->device);
     drop_graphs(h);
     if (h->d_log) {
-        hipFree(h->d_log);
-        h->allocs.erase(std::remove(h->allocs.begin(), h->allocs.end(), (void*)h->d_log), h->allocs.end());
+        dev_free(h, h->d_log);
         h->d_log = nullptr;
     }
     h->log_cap = (unsigned long long)capacity;
