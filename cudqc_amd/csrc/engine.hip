@@ -62,6 +62,13 @@ constexpr int LANE_TASK = 64;  // largest task whose vertices fit a wavefront's 
 // another) run on workgroups of SPLIT_T threads: each step scans the removed vertex's
 // lists, and four times the lanes cut the memory round trips of a long list fourfold.
 constexpr int SPLIT_T = 1024;
+// So do level-0 branches of graphs of at least this many vertices and batches whose largest task
+// has at least as many: there a branch that passes its first bound test recounts thousands of
+// vertices, bound by the loads one workgroup has in flight, and the slowest of them is the
+// launch. R-MAT 2^17 unit 26.5 -> 18.8 ms, 2^18 36.9 -> 27.8 ms, level-0 window of the 2^16
+// graph 4.9 -> 2.3 ms. From 1,000 vertices on it is too early: the 2^15 unit, whose second
+// batch has 11,000 small tasks, goes from 16.3 to 23.4 ms (2,000: 16.4).
+constexpr int WIDE_TASK = 4000;
 #ifndef DQC_SCAN_UNR
 #define DQC_SCAN_UNR 8
 #endif
@@ -1083,6 +1090,7 @@ struct W {
         int removed = ccount - k;
         bool all_mat = (removed == nd);
         while (k > 0 && removed > 0) {
+            if (head_settled()) return false;
             if (all_mat && nd < k + cm) decrement(dropped, nd);
             else recount(cm, cur, k);
             int nv = hist_valid(cur, k, cm, ub, lb, meo, mei);
@@ -2150,6 +2158,13 @@ struct W {
         cand_marks = false;
     }
 
+    // A branch before a level-0 window only tells whether a child is written there: once any
+    // of them has, the others need not finish (all threads agree; asked where a branch is about
+    // to start another long pass).
+    __device__ __forceinline__ bool head_settled() {
+        if (!discard_child) return false;
+        return bcast0(tid == 0 ? __atomic_load_n(&P->q->root_first, __ATOMIC_RELAXED) : 0ull) != ~0ull;
+    }
     // Branch s of the level-0 task, built without replaying the s earlier removals.
     // Level-0 positions are condensed ids and nothing there is a member, so after s
     // removals the live set is [0, k - s), v = k - s - 1, and every value the child
@@ -2157,6 +2172,7 @@ struct W {
     // lvl2adj loses one per removed vertex (id >= k - s) whose two-hop list holds the
     // vertex (reference src/host_functions.cu:1386-1500, 1503-1559).
     __device__ __forceinline__ long long branch_root(int s, int k, const dqc::TaskVertex* root) {
+        if (head_settled()) return -1;
         const int v = k - s - 1, tot = k - s;
         lane_tables = false;
         ptot = l2_tot = tot;  // the values below are computed as of step s
@@ -2972,10 +2988,9 @@ struct W {
         const int chunk = split ? max(1, d.iters) : 1;
         const bool remove_first = piece && (d.flags & TF_REMOVE_FIRST);
         bool first_host_child = (mode == MODE_HOST_L0) && !(d.flags & TF_L1_DONE);
-        if (ROWS && planned)
-            run_chunks(d, tot, ncov, expansions, split, chunk, remove_first, first_host_child, step0);
-        else
-        for (int j = ncov; j < expansions; ++j) {
+        const bool chunked = ROWS && planned;
+        if (chunked) run_chunks(d, tot, ncov, expansions, split, chunk, remove_first, first_host_child, step0);
+        for (int j = chunked ? expansions : ncov; j < expansions; ++j) {
             credit = false;
             // The split pass writes only at chunk starts, so it checks the stack only there:
             // a deferred piece then takes the place of that chunk's piece and no step is
@@ -3160,7 +3175,9 @@ void expand_kernel(KParams P) {
             // level-0 branches keep no live bitmap (the live set is an id range)
             if constexpr (BIG) w.fill_live_summary(~0u);
             w.discard_child = P.split_s[item] < P.root_first;
+            const unsigned long long bytes = w.bytes;
             w.branch_root(P.split_s[item], d.tot, P.in_vtx + d.off);
+            if (w.discard_child) w.bytes = bytes;  // (counts in no statistic)
             w.discard_child = false;
             if constexpr (BIG) w.fill_live_summary(0u);
         } else {
@@ -4442,10 +4459,13 @@ static dqc_status launch(dqc_handle* h, const KParams& P, unsigned long long nta
     unsigned long long gmax = (unsigned long long)(wave ? h->wave_wg : split_pass ? std::min(h->split_wg, h->launch_wg)
                                                                                   : h->launch_wg);
     if (!P.split_s) gmax = std::min(gmax, h->batch_grid);
-    const int grid = (int)std::min<unsigned long long>(gmax, ntask);
+    int grid = (int)std::min<unsigned long long>(gmax, ntask);
+    // large level-0 branches and batches with a large task run on the wide workgroups too
+    const bool wide = split_pass || (!wave && (P.split_s ? h->kloc : (int)std::min<unsigned long long>(h->batch_maxtot, INT_MAX)) >= WIDE_TASK);
+    if (wide) grid = std::min(grid, h->split_wg);
     hipEventRecord(h->ev0, h->stream);
-    if (split_pass && h->big) expand_kernel<true, SPLIT_T><<<grid, SPLIT_T, 0, h->stream>>>(P);
-    else if (split_pass) expand_kernel<false, SPLIT_T><<<grid, SPLIT_T, 0, h->stream>>>(P);
+    if (wide && h->big) expand_kernel<true, SPLIT_T><<<grid, SPLIT_T, 0, h->stream>>>(P);
+    else if (wide) expand_kernel<false, SPLIT_T><<<grid, SPLIT_T, 0, h->stream>>>(P);
     else if (h->big) expand_kernel<true><<<grid, NT, 0, h->stream>>>(P);
     else if (wave) expand_kernel<false, WAVE_T, WAVE_KW><<<grid, WAVE_T, 0, h->stream>>>(P);
     else expand_kernel<false><<<grid, NT, 0, h->stream>>>(P);

@@ -346,7 +346,7 @@ int32_t dqc_generate(int32_t config, int32_t graph_index, const char* path);
  * serving loops, harnesses that forbid hipMalloc. One expansion launch of a batch of
  * tasks, as dqc_step runs it, with every input and output in the caller's device memory
  * and the kernel scratch (launch counters, per-workgroup degree records and lists) in a
- * static device array of the library (about 92 MB per GPU, held until the process
+ * static device array of the library (about 100 MB per GPU, held until the process
  * ends). Nothing is allocated and nothing waits for the host: the launches are queued on
  * `stream` (a hipStream_t; NULL = the null stream) and the outcome lands in `counters`.
  * Limits: condensed graphs of at most DQC_NOALLOC_MAX_VERTICES vertices (larger ones:
