@@ -394,7 +394,10 @@ dqc_status dqc_mlp_train(float* params, const float* x, const float* t, int64_t 
             const int blocks = grad_blocks(m);
             grad_kernel<true><<<blocks, GT>>>(dp, dx, dt, didx + s0, m, 1.f / (float)m, dpart, dl);
             ++step;
-            const float c1 = 1.f - powf(0.9f, (float)step), c2 = 1.f - powf(0.999f, (float)step);
+            // (in double: 1 - 0.999^step cancels, and in float its error, 6e-5 at the first step, was
+            // most of what training was off by)
+            const float c1 = (float)(1.0 - std::pow((double)0.9f, (double)step));
+            const float c2 = (float)(1.0 - std::pow((double)0.999f, (double)step));
             adam_kernel<<<(NPARAM + 63) / 64, 64>>>(dp, dpart, blocks, dm, dv, lr, c1, c2);
         }
         if (hipGetLastError() != hipSuccess) return DQC_E_HIP;
