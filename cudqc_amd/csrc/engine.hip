@@ -1,7 +1,11 @@
 // MI355X (gfx950) expansion engine for maximal directed quasi-clique enumeration.
 //
-// One 256-thread workgroup owns one task at a time and runs its branch loop; the
-// workgroups are persistent and pull tasks from the current batch with one atomic.
+// One workgroup owns one task at a time and runs its branch loop: 256 threads, 1024 for split
+// passes and large tasks, one wavefront for small tasks on small graphs (at most 64
+// vertices: one per lane). The workgroups are persistent and pull tasks from the current
+// batch with one atomic. Where the condensed graph's lists fit as bit rows, 32 loop steps
+// are planned together on those rows and only branches that pass their first bound test
+// touch per-vertex degrees.
 // All tasks live on one LIFO task stack in HBM: each launch expands a batch popped from
 // the stack top, and children are pushed back onto the top with one combined 64-bit
 // atomic per child (descriptor count and record count move together, so the records
@@ -19,7 +23,7 @@
 //     lookup;
 //   * a bitonic sort of each child on a packed 64-bit enumeration-order key, in LDS for
 //     children of up to SORT_N vertices and in the workgroup's HBM area above that (LDS
-//     is kept small so that eight workgroups share a CU).
+//     is kept small so that registers, not LDS, set how many workgroups share a CU: four).
 //
 // Semantics follow the reference's per-task branch loop exactly (host level 0 / 1 or
 // device levels, selected per task); the functions cite the reference lines they follow.
